@@ -217,7 +217,9 @@ int ensure_pinned(cdclq_ctx* ctx, size_t bytes) {
 // ctx->part, then folded in panel order into ctx->G.
 int grad_gemm(cdclq_ctx* ctx, int rows, int n, int c0, int wd, const float* e, const float* h32, const int* rtiles,
               int ntiles) {
-  hipError_t err = panel_gemm(ctx->st, rows, wd, n, e, n, h32 + c0, n, P<float>(ctx->part), rtiles, ntiles);
+  const int ld = repair_ld(n);
+  hipError_t err = panel_gemm(ctx->st, rows, wd, (n + 31) & ~31, e, ld, h32 + c0, ld, P<float>(ctx->part), rtiles,
+                              ntiles);
   if (err == hipSuccess)
     err = fold_panels(ctx->st, rows, wd, (n + 255) / 256, P<float>(ctx->part), P<float>(ctx->G), rtiles, ntiles);
   return err == hipSuccess ? CDCLQ_OK : fail(ctx, CDCLQ_DEVICE, std::string("gradient GEMM: ") + hipGetErrorString(err));
@@ -295,13 +297,15 @@ static int prepare(cdclq_ctx* ctx, const float* w, int d_out, int n, const float
     }
     mean_diag /= (double)n;
     const double damp_val = cfg->damp * mean_diag;
-    CK(ensure(ctx, ctx->cache_h32, (size_t)n * n * 4));
+    const size_t ld = (size_t)repair_ld(n);
+    CK(ensure(ctx, ctx->cache_h32, ld * ld * 4));
     CK(ensure(ctx, ctx->cache_u, (size_t)n * n * 4));
     CK(ensure(ctx, ctx->a64, (size_t)n * n * 8));
     CK(ensure(ctx, ctx->y64, (size_t)n * n * 8));
     {
       PhaseScope ps(ctx, CDCLQ_PHASE_FACTOR);
-      HIPCK(build_flipped(st, n, h, P<uint32_t>(ctx->perm_d), damp_val, P<double>(ctx->a64), P<float>(ctx->cache_h32)));
+      HIPCK(build_flipped(st, n, (int)ld, h, P<uint32_t>(ctx->perm_d), damp_val, P<double>(ctx->a64),
+                          P<float>(ctx->cache_h32)));
       CK(factor(ctx, n, P<double>(ctx->a64), P<double>(ctx->y64), P<float>(ctx->cache_u)));
     }
     ctx->cache_valid = true;
@@ -501,9 +505,16 @@ int quantize_device(cdclq_ctx* ctx, const float* w, size_t d_out_, size_t n_, co
     }
     CK(ensure(ctx, ctx->sel_d, sel.size()));
     HIPCK(hipMemcpyAsync(ctx->sel_d.p, sel.data(), sel.size(), hipMemcpyHostToDevice, st));
-    HIPCK(sub_f32(st, wn, wp, wq, eb));  // e = W - W_hat (src/engine.rs:516-519)
-    const int wdmax = std::max(do_cd ? sbw : 1, do_refit ? g : 1);
-    CK(ensure(ctx, ctx->part, panel_partials_elems(d_out, wdmax, n) * 4));
+    // e = W - W_hat (src/engine.rs:516-519), rows of lde floats (phase 1's errors are done with)
+    const int lde = repair_ld(n), kp = (n + 31) & ~31, np = (n + CDCLQ_KC - 1) / CDCLQ_KC;
+    CK(ensure(ctx, ctx->ebuf, (size_t)d_out * lde * 4));
+    eb = P<float>(ctx->ebuf);
+    HIPCK(residual(st, d_out, n, lde, wp, wq, eb));
+    // steps whose groups / sub-blocks lie inside the KC panels run one panel per launch
+    const bool rpanel = do_refit && refit_panel_ok(n, g), cpanel = do_cd && cd_panel_ok(n, sbw);
+    const int wdmax = std::max(do_cd && !cpanel ? sbw : 1, do_refit && !rpanel ? g : 1);
+    const int wpart = std::max(wdmax, np > 1 && (rpanel || cpanel) ? std::min(lde, CDCLQ_KC) : 1);
+    CK(ensure(ctx, ctx->part, panel_partials_elems(d_out, wpart, n) * 4));
     CK(ensure(ctx, ctx->G, (size_t)d_out * wdmax * 4));
     // Per-pass logs of accepted deltas (folded into the chunk losses in the reference's order).
     const int cap = std::max(1, do_cd ? sbw * (int)cfg->cd_sweeps : 1);
@@ -528,10 +539,17 @@ int quantize_device(cdclq_ctx* ctx, const float* w, size_t d_out_, size_t n_, co
     std::vector<double> prev(nchunks, 0.0);
     std::vector<uint64_t> upd(nchunks);
     // The gradient GEMM runs only over the 128-row tiles that hold rows of a chunk still being
-    // repaired: list 0 for the refit steps (active chunks), list 1 + s for CD sub-block s (active
-    // chunks that selected it). A null list means every tile (the final refit).
+    // repaired: list 0 for the refit steps (active chunks), list 1 + s for the descent's step s, a
+    // sub-block or a panel of spl sub-blocks (active chunks that selected one of them). A null list
+    // means every tile (the final refit).
     const int rt = panel_row_tile(), ntile = (d_out + rt - 1) / rt;
-    std::vector<int> tl((size_t)(1 + n_sb) * ntile), tcnt(1 + n_sb);
+    const int spl = cpanel ? CDCLQ_KC / 64 : 1, ncd = (n_sb + spl - 1) / spl;
+    auto selected = [&](int c, int s) {  // chunk c takes part in descent step s
+      bool any = false;
+      for (int t = s * spl; t < std::min((s + 1) * spl, n_sb) && !any; ++t) any = sel[(size_t)c * n_sb + t];
+      return act[c] && any;
+    };
+    std::vector<int> tl((size_t)(1 + ncd) * ntile), tcnt(1 + ncd);
     const size_t apad = ((size_t)nchunks + 15) / 16 * 16, up_bytes = apad + tl.size() * sizeof(int);
     CK(ensure(ctx, ctx->rtiles_d, up_bytes));
     uint8_t* active = P<uint8_t>(ctx->rtiles_d);
@@ -553,13 +571,13 @@ int quantize_device(cdclq_ctx* ctx, const float* w, size_t d_out_, size_t n_, co
       return CDCLQ_OK;
     };
     auto build_tiles = [&]() -> int {
-      for (int l = 0; l <= n_sb; ++l) {
+      for (int l = 0; l <= ncd; ++l) {
         int cnt = 0;
         for (int t = 0; t < ntile; ++t) {
           const int c_lo = (t * rt) / rc, c_hi = (std::min((t + 1) * rt, d_out) - 1) / rc;
           bool need = false;
           for (int c = c_lo; c <= c_hi && !need; ++c)
-            need = act[c] && (l == 0 || sel[(size_t)c * n_sb + (l - 1)]);
+            need = l == 0 ? act[c] != 0 : selected(c, l - 1);
           if (need) tl[(size_t)l * ntile + cnt++] = t;
         }
         tcnt[l] = cnt;
@@ -570,17 +588,24 @@ int quantize_device(cdclq_ctx* ctx, const float* w, size_t d_out_, size_t n_, co
     bool all_tiles = false;
     auto refit_all = [&]() -> int {
       HIPCK(hipMemsetAsync(rcnt, 0, (size_t)ng * d_out * 4, st));
-      for (int gi = 0; gi < ng; ++gi) {
+      const int* tl0 = all_tiles ? nullptr : rtiles;
+      const int nt0 = all_tiles ? ntile : tcnt[0];
+      for (int q = 0; rpanel && q < np; ++q) {
+        const int c0 = q * CDCLQ_KC, wdp = std::min(lde - c0, CDCLQ_KC);
+        if (np > 1)
+          HIPCK(panel_gemm(st, d_out, wdp, kp, eb, lde, H32 + c0, lde, P<float>(ctx->part), tl0, nt0, q));
+        HIPCK(refit_panel(st, RefitPanelArgs{d_out, n, lde, ng, g, q, rc, np, wdp, P<float>(ctx->part), H32, codes,
+                                             scales, zeros, wq, eb, active, rlog, rcnt}));
+      }
+      for (int gi = 0; !rpanel && gi < ng; ++gi) {
         const int c0 = gi * g, wd = std::min(c0 + g, n) - c0;
-        const int* tl0 = all_tiles ? nullptr : rtiles;
-        const int nt0 = all_tiles ? ntile : tcnt[0];
         // the refit kernel folds the per-panel chains itself where it can (one launch less)
         const bool fused = refit_folds_chains(wd);
         if (fused)
-          HIPCK(panel_gemm(st, d_out, wd, n, eb, n, H32 + c0, n, P<float>(ctx->part), tl0, nt0));
+          HIPCK(panel_gemm(st, d_out, wd, kp, eb, lde, H32 + c0, lde, P<float>(ctx->part), tl0, nt0));
         else
           CK(grad_gemm(ctx, d_out, n, c0, wd, eb, H32, tl0, nt0));
-        HIPCK(refit_group(st, d_out, n, ng, g, gi, rc, P<float>(ctx->G), H32, codes, scales, zeros, wq, eb,
+        HIPCK(refit_group(st, d_out, n, lde, ng, g, gi, rc, P<float>(ctx->G), H32, codes, scales, zeros, wq, eb,
                           active, rlog + (size_t)gi * d_out, rcnt + (size_t)gi * d_out,
                           fused ? P<float>(ctx->part) : nullptr, fused ? (n + 255) / 256 : 0));
       }
@@ -592,19 +617,26 @@ int quantize_device(cdclq_ctx* ctx, const float* w, size_t d_out_, size_t n_, co
       if (do_refit) CK(refit_all());
       if (do_cd) {
         HIPCK(hipMemsetAsync(ccnt, 0, (size_t)n_sb * d_out * 4, st));
-        for (int s = 0; s < n_sb; ++s) {
-          bool any = false;
-          for (int c = 0; c < nchunks && !any; ++c) any = act[c] && sel[(size_t)c * n_sb + s];
-          if (!any) continue;
-          const int c0 = s * sbw, wd = std::min(c0 + sbw, n) - c0;
+        for (int s = 0; s < ncd; ++s) {
+          if (tcnt[1 + s] == 0) continue;
           const int* tl_s = rtiles + (size_t)(1 + s) * ntile;
+          if (cpanel) {
+            const int c0 = s * CDCLQ_KC, wdp = std::min(lde - c0, CDCLQ_KC);
+            if (np > 1)
+              HIPCK(panel_gemm(st, d_out, wdp, kp, eb, lde, H32 + c0, lde, P<float>(ctx->part), tl_s, tcnt[1 + s], s));
+            HIPCK(cd_panel(st, CdPanelArgs{d_out, n, lde, ng, g, s, n_sb, rc, (int)cfg->cd_sweeps, cap, np, wdp,
+                                           P<float>(ctx->part), H32, P<uint8_t>(ctx->gbits_d), scales, zeros, codes,
+                                           wq, eb, active, P<uint8_t>(ctx->sel_d), clog, ccnt, mid, cd_evals}));
+            continue;
+          }
+          const int c0 = s * sbw, wd = std::min(c0 + sbw, n) - c0;
           // the descent kernel folds the per-panel chains itself where it can (one launch less)
           const bool fused = cd_folds_chains(wd);
           if (fused)
-            HIPCK(panel_gemm(st, d_out, wd, n, eb, n, H32 + c0, n, P<float>(ctx->part), tl_s, tcnt[1 + s]));
+            HIPCK(panel_gemm(st, d_out, wd, kp, eb, lde, H32 + c0, lde, P<float>(ctx->part), tl_s, tcnt[1 + s]));
           else
             CK(grad_gemm(ctx, d_out, n, c0, wd, eb, H32, tl_s, tcnt[1 + s]));
-          HIPCK(cd_subblock(st, d_out, n, ng, g, c0, wd, s, n_sb, rc, (int)cfg->cd_sweeps, P<float>(ctx->G), H32,
+          HIPCK(cd_subblock(st, d_out, n, lde, ng, g, c0, wd, s, n_sb, rc, (int)cfg->cd_sweeps, P<float>(ctx->G), H32,
                             P<uint8_t>(ctx->gbits_d), scales, zeros, codes, wq, eb, active,
                             P<uint8_t>(ctx->sel_d), clog + (size_t)s * d_out * cap, ccnt + (size_t)s * d_out, cap,
                             mid, cd_evals, fused ? P<float>(ctx->part) : nullptr, fused ? (n + 255) / 256 : 0));

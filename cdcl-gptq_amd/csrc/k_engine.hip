@@ -565,6 +565,16 @@ __global__ __launch_bounds__(256) void k_colloss(int rows, int n, int rc, const 
   out[(long)c * n + j] = s;
 }
 
+// e = a - b (rows x n), rows of ld floats zero past column n
+__global__ __launch_bounds__(256) void k_residual(int rows, int n, int ld, const float* __restrict__ a,
+                                                  const float* __restrict__ b, float* __restrict__ e) {
+  const long idx = (long)blockIdx.x * 256 + threadIdx.x;
+  if (idx >= (long)rows * ld) return;
+  const int r = (int)(idx / ld), c = (int)(idx % ld);
+  const long o = (long)r * n + c;
+  e[idx] = c < n ? a[o] - b[o] : 0.0f;
+}
+
 __global__ __launch_bounds__(256) void k_sub(long count, const float* __restrict__ a, const float* __restrict__ b,
                                              float* __restrict__ o) {
   const long idx = (long)blockIdx.x * 256 + threadIdx.x;
@@ -834,6 +844,11 @@ hipError_t gptq_block(hipStream_t st, int rows, int n, int i1, int cnt, int g, i
 hipError_t colloss(hipStream_t st, int rows, int n, int rc, const float* err, double* out) {
   const int nchunks = (rows + rc - 1) / rc;
   hipLaunchKernelGGL(k_colloss, dim3(nblk(n), nchunks), dim3(256), 0, st, rows, n, rc, err, out);
+  return hipGetLastError();
+}
+
+hipError_t residual(hipStream_t st, int rows, int n, int ld, const float* a, const float* b, float* e) {
+  hipLaunchKernelGGL(k_residual, dim3(nblk((long)rows * ld)), dim3(256), 0, st, rows, n, ld, a, b, e);
   return hipGetLastError();
 }
 

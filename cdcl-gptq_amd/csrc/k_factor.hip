@@ -19,12 +19,17 @@ namespace {
 constexpr int NBC = 96;  // src/linalg.rs:202, :285
 
 // hp = perm(H) in f64, dead diagonal -> 1, + damp on the diagonal; h32 = (f32)hp; a = flip(hp).
-__global__ __launch_bounds__(256) void k_build_flipped(int n, const float* __restrict__ h,
+// h32 is ld x ld, zero past n.
+__global__ __launch_bounds__(256) void k_build_flipped(int n, int ld, const float* __restrict__ h,
                                                        const uint32_t* __restrict__ perm, double damp_val,
                                                        double* __restrict__ a, float* __restrict__ h32) {
   const long idx = (long)blockIdx.x * 256 + threadIdx.x;
-  if (idx >= (long)n * n) return;
-  const int p = (int)(idx / n), q = (int)(idx % n);
+  if (idx >= (long)ld * ld) return;
+  const int p = (int)(idx / ld), q = (int)(idx % ld);
+  if (p >= n || q >= n) {
+    h32[idx] = 0.0f;
+    return;
+  }
   double v = (double)h[(long)perm[p] * n + perm[q]];
   if (p == q) {
     if (v == 0.0) v = 1.0;
@@ -309,9 +314,9 @@ inline unsigned nblk(long count) { return (unsigned)((count + 255) / 256); }
 
 }  // namespace
 
-hipError_t build_flipped(hipStream_t st, int n, const float* h, const uint32_t* perm, double damp_val, double* a,
-                         float* h32) {
-  hipLaunchKernelGGL(k_build_flipped, dim3(nblk((long)n * n)), dim3(256), 0, st, n, h, perm, damp_val, a, h32);
+hipError_t build_flipped(hipStream_t st, int n, int ld, const float* h, const uint32_t* perm, double damp_val,
+                         double* a, float* h32) {
+  hipLaunchKernelGGL(k_build_flipped, dim3(nblk((long)ld * ld)), dim3(256), 0, st, n, ld, h, perm, damp_val, a, h32);
   return hipGetLastError();
 }
 

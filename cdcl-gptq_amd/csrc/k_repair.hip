@@ -1,14 +1,13 @@
 // Phase-2 kernels (src/engine.rs:534-670): the repair gradient G = E H[:, c0:c0+wd] on the matrix
-// cores, and the refit / coordinate-descent sweeps that consume it.
+// cores, and the refit / coordinate-descent sweeps of groups and sub-blocks that do not lie inside
+// the KC panels (the others run a panel per launch, k_panel.hip).
 //
 // Gradient. The reference computes G with matrixmultiply (k = n): per element a fused chain over
-// each KC = 256 panel of k, panels folded in order. k_panel_gemm computes every panel's chain in
+// each KC = 256 panel of k, panels folded in order. The GEMMs compute the panels' chains in
 // parallel with v_mfma_f32_32x32x1_2b_f32 (K = 1, single rounding per product, bit-identical to
-// fmaf) and stores the per-panel values; k_fold then folds them in panel order, one thread per
-// element. Workgroup: 128 rows x 64 cols x one panel, E and the panel of H staged in
-// double-buffered LDS.
+// fmaf) and store the per-panel values; the sweeps (or k_fold) fold them in panel order.
 //
-// Sweeps. The refit of a group of at most 128 columns computes U H_CC for 64 rows on the matrix
+// Sweeps. The refit of a group of at most 128 columns computes U H_CC for 16-64 rows on the matrix
 // cores from H_CC staged in LDS (wider groups: one wavefront per row, H_CC from L2). The descent
 // runs one wavefront per row, columns over lanes: it evaluates all columns of a sub-block at once
 // and touches a row of H_sb only when a code moves, reading it from L2.
@@ -45,7 +44,7 @@ __device__ __forceinline__ v32f mfma32(float a, float b, v32f c) {
 // pipeline runs across unit boundaries: the first stage of the next unit is loaded while the last
 // stage of the current one is multiplied, and the accumulator is written out and cleared between
 // them, so no workgroup pays a cold start per panel.
-template <int SK, bool VEC4>
+template <int SK>
 __global__ __launch_bounds__(256) void k_panel_gemm(int m, int wd, int k, const float* __restrict__ A, long lda,
                                                     const float* __restrict__ B, long ldb, float* __restrict__ P,
                                                     int nunits, const int* __restrict__ rtiles, int nrt) {
@@ -76,26 +75,14 @@ __global__ __launch_bounds__(256) void k_panel_gemm(int m, int wd, int k, const 
     return t;
   };
   float4 pe[EQ], ph[HQ];
-  // VEC4: unconditional 16-byte loads from clamped addresses (rows >= m only feed outputs that are
-  // never stored; k slots past the panel are replaced below); otherwise guarded scalar loads.
+  // E: unconditional 16-byte loads from clamped addresses (rows >= m only feed outputs that are
+  // never stored; k slots past the panel are replaced below). B: guarded scalar loads.
   auto gload = [&](const Unit& t, int ks) {
 #pragma unroll
     for (int q = 0; q < EQ; ++q) {
       const int e = tid + 256 * q;
       const int r = t.r0 + e / K4, kk = ks + (e % K4) * 4;
-      if (VEC4) {
-        pe[q] = *reinterpret_cast<const float4*>(A + (long)min(r, m - 1) * lda + t.k0 + min(kk, t.kc - 4));
-      } else {
-        float4 v = make_float4(-0.f, -0.f, -0.f, -0.f);
-        if (r < m) {
-          const float* src = A + (long)r * lda + t.k0 + kk;
-          if (kk < t.kc) v.x = src[0];
-          if (kk + 1 < t.kc) v.y = src[1];
-          if (kk + 2 < t.kc) v.z = src[2];
-          if (kk + 3 < t.kc) v.w = src[3];
-        }
-        pe[q] = v;
-      }
+      pe[q] = *reinterpret_cast<const float4*>(A + (long)min(r, m - 1) * lda + t.k0 + min(kk, t.kc - 4));
     }
 #pragma unroll
     for (int q = 0; q < HQ; ++q) {
@@ -117,10 +104,10 @@ __global__ __launch_bounds__(256) void k_panel_gemm(int m, int wd, int k, const 
     for (int q = 0; q < EQ; ++q) {
       const int e = tid + 256 * q;
       float4 v = pe[q];
-      // k is a multiple of 4 under VEC4, so a slot is either wholly inside the panel or wholly past
+      // k is a multiple of 4, so a slot is either wholly inside the panel or wholly past
       // its end (then the clamped load read other data). Past the end, E is -0 and B is +0: the
       // step fma(-0, +0, c) = c + (-0) = c leaves every chain value unchanged, -0 included.
-      if (VEC4 && ks + (e % K4) * 4 >= t.kc) v = make_float4(-0.f, -0.f, -0.f, -0.f);
+      if (ks + (e % K4) * 4 >= t.kc) v = make_float4(-0.f, -0.f, -0.f, -0.f);
       *reinterpret_cast<float4*>(&Es[buf][(e / K4) * ES + (e % K4) * 4]) = v;
     }
 #pragma unroll
@@ -179,8 +166,8 @@ __global__ __launch_bounds__(256) void k_panel_gemm(int m, int wd, int k, const 
   }
 }
 
-// Direct-to-LDS variant of k_panel_gemm, used when k % 32 == 0, wd % 4 == 0 and the rows of E and
-// H are 16-byte aligned. Stages are filled with global_load_lds_dwordx4 into a ring of three, two
+// Direct-to-LDS form, used when k % 32 == 0, wd % 4 == 0 and the rows of E and H are 16-byte
+// aligned (k_panel_gemm takes the rest). Stages are filled with global_load_lds_dwordx4 into a ring of three, two
 // stages in flight behind the one being multiplied, one bare barrier per stage; units, the MFMA
 // mapping and the outputs are those of k_panel_gemm. Stage layout: E as [128 rows][8 slots][4],
 // slot s of row r holding k-quad s ^ (r & 7) (load i: lane l -> row 8 i + (l >> 3), so each load
@@ -205,9 +192,10 @@ __global__ __launch_bounds__(256) void k_panel_dma(int m, int wd, int k, const f
                                                    const float* __restrict__ B, long ldb, float* __restrict__ P,
                                                    int nunits, const int* __restrict__ rtiles, int nrt,
                                                    float* __restrict__ C, long ldc, float alpha, int beta_one,
-                                                   int kfold) {
+                                                   int kfold, int skip) {
   __shared__ float R[DNB][DSTAGE];
-  const int np = k / CDCLQ_KC + (k % CDCLQ_KC != 0);
+  const int nct = (wd + PC - 1) / PC;
+  const int np = k / CDCLQ_KC + (k % CDCLQ_KC != 0) - (skip >= 0);  // panels computed
   // With a full grid (two workgroups per CU), workgroups j and j + G/2 end up on the same CU: the
   // first half fills every CU once and the second half pairs up with it in dispatch order. They
   // take adjacent unit ranges 2j and 2j + 1, whose sizes (floor and ceiling of units / G) add up
@@ -225,18 +213,17 @@ __global__ __launch_bounds__(256) void k_panel_dma(int m, int wd, int k, const f
   auto unit = [&](int u) {
     Unit t;
     if (DIRECT) {  // all of k; column tiles fastest, so consecutive units share their E tile
-      const int nct = (wd + PC - 1) / PC;
       t.r0 = (u / nct) * PR;
       t.cb = (u % nct) * PC;
       t.p = 0;
       t.k0 = 0;
       t.nst = k / DSK;
-    } else {
-      const int ct = u / (nrt * np), rem = u % (nrt * np);
+    } else {  // (row tile, panel, column tile), column tiles fastest
+      const int ct = u % nct, rem = u / nct;
       t.r0 = (rtiles ? rtiles[rem / np] : rem / np) * PR;
       t.p = rem % np;
       t.cb = ct * PC;
-      t.k0 = t.p * CDCLQ_KC;
+      t.k0 = (t.p + (skip >= 0 && t.p >= skip)) * CDCLQ_KC;
       t.nst = min(CDCLQ_KC, k - t.k0) / DSK;
     }
     return t;
@@ -402,14 +389,14 @@ template <bool DIRECT>
 __global__ __launch_bounds__(512) void k_lazy_wide(int m, int wd, int k, const float* __restrict__ A, long lda,
                                                    const float* __restrict__ B, long ldb, float* __restrict__ C,
                                                    long ldc, float alpha, int nunits, float* __restrict__ P,
-                                                   const int* __restrict__ rtiles, int kfold) {
+                                                   const int* __restrict__ rtiles, int kfold, int skip) {
   // With C a ring of two stages (64 KB), so that a narrow update's workgroup (72 KB) fits beside
   // this one on each CU: this kernel runs on a side stream while the main stream updates and
   // sweeps the next blocks. Without C the ring of three.
   constexpr int NB = DIRECT ? 2 : DNB;
   __shared__ float R[NB][LSTAGE];
   const int nct = (wd + LPC - 1) / LPC;
-  const int np = k / CDCLQ_KC + (k % CDCLQ_KC != 0);
+  const int np = k / CDCLQ_KC + (k % CDCLQ_KC != 0) - (skip >= 0);  // panels computed
   const int u0 = (int)((long)blockIdx.x * nunits / gridDim.x);
   const int u1 = (int)((long)(blockIdx.x + 1) * nunits / gridDim.x);
   if (u0 >= u1) return;
@@ -427,11 +414,12 @@ __global__ __launch_bounds__(512) void k_lazy_wide(int m, int wd, int k, const f
       t.p = 0;
       t.k0 = 0;
       t.nst = k / DSK;
-    } else {  // the repair gradient, wd == 128: (row tile, panel), panels fastest
-      t.r0 = (rtiles ? rtiles[u / np] : u / np) * PR;
-      t.cb = 0;
-      t.p = u % np;
-      t.k0 = t.p * CDCLQ_KC;
+    } else {  // the repair gradient: (row tile, panel, column tile), column tiles fastest
+      const int rem = u / nct;
+      t.r0 = (rtiles ? rtiles[rem / np] : rem / np) * PR;
+      t.cb = (u % nct) * LPC;
+      t.p = rem % np;
+      t.k0 = (t.p + (skip >= 0 && t.p >= skip)) * CDCLQ_KC;
       t.nst = min(CDCLQ_KC, k - t.k0) / DSK;
     }
     return t;
@@ -489,8 +477,8 @@ __global__ __launch_bounds__(512) void k_lazy_wide(int m, int wd, int k, const f
   // as in k_panel_dma: a whole tile stores from one address per lane plus uniform offsets
   auto roff = [](int r, long ld) { return ((r & 3) + 8 * ((r & 15) >> 2)) * ld + 32 * (r >> 4); };
   auto store_p = [&](const Unit& t) {
-    if (t.r0 + PR <= m && LPC <= wd) {
-      float* q = P + ((long)t.p * m + t.r0 + 32 * wr + 4 * (lane >> 5)) * wd + 64 * wc + (lane & 31);
+    if (t.r0 + PR <= m && t.cb + LPC <= wd) {
+      float* q = P + ((long)t.p * m + t.r0 + 32 * wr + 4 * (lane >> 5)) * wd + t.cb + 64 * wc + (lane & 31);
 #pragma unroll
       for (int r = 0; r < 32; ++r) __builtin_nontemporal_store(acc[r], q + roff(r, wd));
       return;
@@ -498,7 +486,7 @@ __global__ __launch_bounds__(512) void k_lazy_wide(int m, int wd, int k, const f
 #pragma unroll
     for (int r = 0; r < 32; ++r) {
       const int row = t.r0 + 32 * wr + (r & 3) + 8 * ((r & 15) >> 2) + 4 * (lane >> 5);
-      const int col = 64 * wc + 32 * (r >> 4) + (lane & 31);
+      const int col = t.cb + 64 * wc + 32 * (r >> 4) + (lane & 31);
       if (row < m && col < wd) __builtin_nontemporal_store(acc[r], &P[((long)t.p * m + row) * wd + col]);
     }
   };
@@ -601,7 +589,7 @@ __global__ __launch_bounds__(256) void k_fold(int m, int wd, int np, const int* 
 // columns (narrower ones take k_refit_mfma). One wavefront per row, columns over lanes; H_CC is
 // read from L2.
 template <int NPL>
-__global__ __launch_bounds__(256) void k_refit(int rows, int n, int ng, int g, int gi, int rc, const float* __restrict__ G,
+__global__ __launch_bounds__(256) void k_refit(int rows, int n, int ld, int ng, int g, int gi, int rc, const float* __restrict__ G,
                                                const float* __restrict__ h32,
                                                const uint8_t* __restrict__ codes, float* __restrict__ scales,
                                                const float* __restrict__ zeros, float* __restrict__ wq,
@@ -643,7 +631,7 @@ __global__ __launch_bounds__(256) void k_refit(int rows, int n, int ng, int g, i
 #pragma unroll
     for (int s2 = 0; s2 < NPL; ++s2) {
       const int k2 = s2 * 64 + lane;
-      h[s2] = k2 < wd ? h32[(long)(c0 + k) * n + c0 + k2] : 0.0f;
+      h[s2] = k2 < wd ? h32[(long)(c0 + k) * ld + c0 + k2] : 0.0f;
     }
 #pragma unroll
     for (int q = 0; q < RW; ++q) {
@@ -724,9 +712,9 @@ __global__ __launch_bounds__(256) void k_refit(int rows, int n, int ng, int g, i
         for (int s = 0; s < NPL; ++s) {
           const int k = s * 64 + lane;
           if (k < wd) {
-            const long o = (long)r * n + c0 + k;
+            const long o = (long)r * n + c0 + k, oe = (long)r * ld + c0 + k;
             const float ndq = s_new * uu[q][s];
-            e[o] = e[o] + (wq[o] - ndq);
+            e[oe] = e[oe] + (wq[o] - ndq);
             wq[o] = ndq;
           }
         }
@@ -758,7 +746,7 @@ __device__ __forceinline__ v16f mfma16(float a, float b, v16f c) {
 }
 
 template <int RF_ROWS>
-__global__ __launch_bounds__(256) void k_refit_mfma(int rows, int n, int ng, int g, int gi, int rc,
+__global__ __launch_bounds__(256) void k_refit_mfma(int rows, int n, int ld, int ng, int g, int gi, int rc,
                                                     const float* __restrict__ G, const float* __restrict__ h32,
                                                     const uint8_t* __restrict__ codes, float* __restrict__ scales,
                                                     const float* __restrict__ zeros, float* __restrict__ wq,
@@ -818,7 +806,7 @@ __global__ __launch_bounds__(256) void k_refit_mfma(int rows, int n, int ng, int
 #pragma unroll
     for (int u = 0; u < 16; ++u) {
       const int x = tid + 256 * u;  // float4 slot: row x >> 5, columns 4 (x & 31) ..
-      hq[u] = *reinterpret_cast<const v4f*>(h32 + (long)(c0 + (x >> 5)) * n + c0 + 4 * (x & 31));
+      hq[u] = *reinterpret_cast<const v4f*>(h32 + (long)(c0 + (x >> 5)) * ld + c0 + 4 * (x & 31));
     }
 #pragma unroll
     for (int u = 0; u < RF_ROWS * 32 / 256; ++u) {
@@ -845,7 +833,7 @@ __global__ __launch_bounds__(256) void k_refit_mfma(int rows, int n, int ng, int
 #pragma unroll
       for (int u = 0; u < BATCH; ++u) {
         const int x = tid + 256 * (b + u);
-        v[u] = h32[(long)(c0 + min(x >> 7, wd - 1)) * n + c0 + min(x & 127, wd - 1)];
+        v[u] = h32[(long)(c0 + min(x >> 7, wd - 1)) * ld + c0 + min(x & 127, wd - 1)];
       }
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -1063,7 +1051,7 @@ __global__ __launch_bounds__(256) void k_refit_mfma(int rows, int n, int ng, int
       const int x = tid + 256 * i, rl = x >> 5, k4 = x & 31;
       if (mv[rl]) {
         const long o = (long)(r0 + rl) * n + c0 + 4 * k4;
-        ev[i] = *reinterpret_cast<const v4f*>(e + o);
+        ev[i] = *reinterpret_cast<const v4f*>(e + (long)(r0 + rl) * ld + c0 + 4 * k4);
         qv[i] = *reinterpret_cast<const v4f*>(wq + o);
       }
     }
@@ -1079,7 +1067,7 @@ __global__ __launch_bounds__(256) void k_refit_mfma(int rows, int n, int ng, int
           nq[j] = snew[rl] * ((float)((cw >> (8 * j)) & 0xffu) - zrow[rl]);
           ne[j] = ev[i][j] + (qv[i][j] - nq[j]);
         }
-        *reinterpret_cast<v4f*>(e + o) = ne;
+        *reinterpret_cast<v4f*>(e + (long)(r0 + rl) * ld + c0 + 4 * k4) = ne;
         *reinterpret_cast<v4f*>(wq + o) = nq;
       }
     }
@@ -1095,7 +1083,7 @@ __global__ __launch_bounds__(256) void k_refit_mfma(int rows, int n, int ng, int
       const int x = tid + 256 * (PER * h + i), rl = x >> 7, k = x & 127;
       if (k < wd && mv[rl]) {
         const long o = (long)(r0 + rl) * n + c0 + k;
-        ev[i] = e[o];
+        ev[i] = e[(long)(r0 + rl) * ld + c0 + k];
         qv[i] = wq[o];
       }
     }
@@ -1105,7 +1093,7 @@ __global__ __launch_bounds__(256) void k_refit_mfma(int rows, int n, int ng, int
       if (k < wd && mv[rl]) {
         const long o = (long)(r0 + rl) * n + c0 + k;
         const float ndq = snew[rl] * ((float)cb[rl * RF_CS + k] - zrow[rl]);
-        e[o] = ev[i] + (qv[i] - ndq);
+        e[(long)(r0 + rl) * ld + c0 + k] = ev[i] + (qv[i] - ndq);
         wq[o] = ndq;
       }
     }
@@ -1158,7 +1146,7 @@ template <int NPL, int FBW = 0>
 // otherwise take enough scalar registers to cap it at 7. FBW (64-column form only) widens the
 // fold's batches to FBW panels for gradients of many panels, at 6 wavefronts per SIMD.
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NPL == 1 ? (FBW ? 6 : 8) : 1))) void k_cd(
-    int rows, int n, int ng, int g, int c0, int wd, int sb, int nsb, int rc, int sweeps, const float* __restrict__ G,
+    int rows, int n, int ld, int ng, int g, int c0, int wd, int sb, int nsb, int rc, int sweeps, const float* __restrict__ G,
     const float* __restrict__ h32, const uint8_t* __restrict__ gbits, const float* __restrict__ scales,
     const float* __restrict__ zeros, uint8_t* __restrict__ codes, float* __restrict__ wq, float* __restrict__ e,
     const uint8_t* __restrict__ active, const uint8_t* __restrict__ sel, double* __restrict__ dlog,
@@ -1178,7 +1166,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NPL == 1 ? 
 #pragma unroll
     for (int q = 0; q < HPER; ++q) {
       const int x = threadIdx.x + 256 * q, i = x / HW, c = x % HW;
-      hv[q] = h32[(long)(c0 + min(i, wd - 1)) * n + c0 + min(c, wd - 1)];
+      hv[q] = h32[(long)(c0 + min(i, wd - 1)) * ld + c0 + min(c, wd - 1)];
     }
   }
   const int chunk = min(r, rows - 1) / rc;
@@ -1198,9 +1186,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NPL == 1 ? 
       const long o = (long)r * n + j;
       const int gi = j / g;
       mwq[s] = wq[o];
-      me[s] = e[o];
+      me[s] = e[(long)r * ld + j];
       mc[s] = (int)codes[o];
-      hd[s] = h32[(long)j * n + j];
+      hd[s] = h32[(long)j * ld + j];
       sc[s] = scales[(long)r * ng + gi];
       zz[s] = zeros[(long)r * ng + gi];
       gb[s] = gbits[gi];
@@ -1260,7 +1248,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NPL == 1 ? 
         const float d32 = (2.0f * de) * gj + (de * de) * hjj;
         if (lane == 0) dl[moves] = (double)d32;
         ++moves;
-        const float* hrow = HLDS ? &hs[(s * 64 + jl) * HW] : h32 + (long)(c0 + s * 64 + jl) * n + c0;
+        const float* hrow = HLDS ? &hs[(s * 64 + jl) * HW] : h32 + (long)(c0 + s * 64 + jl) * ld + c0;
 #pragma unroll
         for (int s2 = 0; s2 < NPL; ++s2) {  // lanes past wd (never selected, never stored) take
           const int k = s2 * 64 + lane;       // garbage: no predicate, clamped address
@@ -1283,7 +1271,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NPL == 1 ? 
     if (k < wd) {
       const long o = (long)r * n + c0 + k;
       wq[o] = mwq[s];
-      e[o] = me[s];
+      e[(long)r * ld + c0 + k] = me[s];
       codes[o] = (uint8_t)mc[s];
     }
   }
@@ -1299,7 +1287,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NPL == 1 ? 
 // buffer, updated in place) and the per-column state in wq / e / codes, visited 64 columns at a
 // time. After a move the whole gradient row is updated in memory and the current slice reloaded;
 // a workgroup-scope fence orders the wave's stores before its next loads.
-__global__ __launch_bounds__(256) void k_cd_mem(int rows, int n, int ng, int g, int c0, int wd, int sb, int nsb,
+__global__ __launch_bounds__(256) void k_cd_mem(int rows, int n, int ld, int ng, int g, int c0, int wd, int sb, int nsb,
                                                 int rc, int sweeps, float* __restrict__ G,
                                                 const float* __restrict__ h32, const uint8_t* __restrict__ gbits,
                                                 const float* __restrict__ scales, const float* __restrict__ zeros,
@@ -1327,9 +1315,9 @@ __global__ __launch_bounds__(256) void k_cd_mem(int rows, int n, int ng, int g, 
       const int j = c0 + min(k, wd - 1);
       const long o = (long)r * n + j;
       const int gi = j / g;
-      const float hd = h32[(long)j * n + j], sc = scales[(long)r * ng + gi], zz = zeros[(long)r * ng + gi];
+      const float hd = h32[(long)j * ld + j], sc = scales[(long)r * ng + gi], zz = zeros[(long)r * ng + gi];
       const float mq = (float)((1u << gbits[gi]) - 1u);
-      float mwq = in ? wq[o] : 0.0f, me = in ? e[o] : 0.0f;
+      float mwq = in ? wq[o] : 0.0f, me = in ? e[(long)r * ld + j] : 0.0f;
       int mc = in ? (int)codes[o] : 0;
       float gg = in ? gr[k] : 0.0f;
       const uint64_t inmask = __ballot(in);
@@ -1359,11 +1347,11 @@ __global__ __launch_bounds__(256) void k_cd_mem(int rows, int n, int ng, int g, 
           mc = qc;
           me = me + de;
           wq[o] = mwq;
-          e[o] = me;
+          e[(long)r * ld + j] = me;
           codes[o] = (uint8_t)mc;
         }
         // g_k = g_k + de * H[j, c0 + k] over the whole sub-block row (src/engine.rs:641-646)
-        const float* hrow = h32 + (long)(c0 + s0 + jl) * n + c0;
+        const float* hrow = h32 + (long)(c0 + s0 + jl) * ld + c0;
         for (int k2 = lane; k2 < wd; k2 += 64) gr[k2] = gr[k2] + de * hrow[k2];
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
         gg = in ? gr[k] : 0.0f;
@@ -1397,8 +1385,7 @@ size_t panel_partials_elems(int m, int wd, int k) {
 
 int panel_row_tile() { return PR; }
 
-// compute units of the current device (cached per process)
-static hipError_t cu_count(int* out) {
+hipError_t device_cus(int* out) {
   static std::atomic<int> cached{0};
   int v = cached.load(std::memory_order_relaxed);
   if (v == 0) {
@@ -1449,55 +1436,51 @@ static hipError_t wide_slots(int* out) {
 }
 
 hipError_t panel_gemm(hipStream_t st, int m, int wd, int k, const float* A, long lda, const float* B, long ldb,
-                      float* P, const int* rtiles, int ntiles) {
+                      float* P, const int* rtiles, int ntiles, int skip) {
   if (m <= 0 || wd <= 0 || k <= 0) return hipSuccess;
   if (!rtiles) ntiles = (m + PR - 1) / PR;
   if (ntiles <= 0) return hipSuccess;
-  const bool vec4 = (lda % 4 == 0) && ((uintptr_t)A % 16 == 0) && k % 4 == 0;
-  constexpr int SK = 32;
-  const long nunits = (long)ntiles * ((k + CDCLQ_KC - 1) / CDCLQ_KC) * ((wd + PC - 1) / PC);
-  if (nunits > INT32_MAX) return hipErrorInvalidValue;
-  // one workgroup per resident slot (occupancy is a property of the kernel, cached per process;
-  // concurrent first calls compute the same value)
-  static std::atomic<int> slots[2] = {0, 0};
-  std::atomic<int>& sl = slots[vec4 ? 1 : 0];
-  if (sl.load(std::memory_order_relaxed) == 0) {
-    int dev = 0, cus = 0, per = 0;
-    hipError_t err = hipGetDevice(&dev);
-    if (err == hipSuccess) err = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    if (err == hipSuccess)
-      err = vec4 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_panel_gemm<SK, true>, 256, 0)
-                 : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_panel_gemm<SK, false>, 256, 0);
-    if (err != hipSuccess) return err;
-    sl.store(std::max(1, cus * std::max(1, per)), std::memory_order_relaxed);
-  }
-  const int grid = (int)std::min<long>(nunits, sl.load(std::memory_order_relaxed));
-  const bool dma = vec4 && k % DSK == 0 && wd % 4 == 0 && wd >= 4 && ldb % 4 == 0 && (uintptr_t)B % 16 == 0;
+  if (lda % 4 != 0 || (uintptr_t)A % 16 != 0 || k % 4 != 0) return hipErrorInvalidValue;  // (the engine's E always is)
+  const bool dma = k % DSK == 0 && wd % 4 == 0 && wd >= 4 && ldb % 4 == 0 && (uintptr_t)B % 16 == 0;
   if (dma) {
-    if (wd == LPC) {  // 128-column gradients of tall enough matrices: one E tile read per unit
+    const long np = (k + CDCLQ_KC - 1) / CDCLQ_KC - (skip >= 0 ? 1 : 0);
+    const long wunits = (long)ntiles * np * ((wd + LPC - 1) / LPC), dunits = (long)ntiles * np * ((wd + PC - 1) / PC);
+    if (dunits == 0) return hipSuccess;
+    if (dunits > INT32_MAX) return hipErrorInvalidValue;
+    if (wd >= LPC) {  // 128-column tiles where there are enough: one E tile read per unit
       int ws = 0;
       const hipError_t e2 = wide_slots<false>(&ws);
       if (e2 != hipSuccess) return e2;
-      const long wunits = (long)ntiles * ((k + CDCLQ_KC - 1) / CDCLQ_KC);
       if (wunits >= 4L * ws) {
         hipLaunchKernelGGL(k_lazy_wide<false>, dim3(ws), dim3(512), 0, st, m, wd, k, A, lda, B, ldb, (float*)nullptr,
-                           0L, 0.0f, (int)wunits, P, rtiles, CDCLQ_KC);
+                           0L, 0.0f, (int)wunits, P, rtiles, CDCLQ_KC, skip);
         return hipGetLastError();
       }
     }
     int dslots = 0;
     const hipError_t err = dma_slots(&dslots);
     if (err != hipSuccess) return err;
-    hipLaunchKernelGGL(k_panel_dma<false>, dim3((int)std::min<long>(nunits, dslots)), dim3(256), 0, st, m, wd, k, A, lda,
-                       B, ldb, P, (int)nunits, rtiles, ntiles, (float*)nullptr, 0L, 0.0f, 0, CDCLQ_KC);
+    hipLaunchKernelGGL(k_panel_dma<false>, dim3((int)std::min<long>(dunits, dslots)), dim3(256), 0, st, m, wd, k, A, lda,
+                       B, ldb, P, (int)dunits, rtiles, ntiles, (float*)nullptr, 0L, 0.0f, 0, CDCLQ_KC, skip);
     return hipGetLastError();
   }
-  if (vec4)
-    hipLaunchKernelGGL((k_panel_gemm<SK, true>), dim3(grid), dim3(256), 0, st, m, wd, k, A, lda, B, ldb, P,
-                       (int)nunits, rtiles, ntiles);
-  else
-    hipLaunchKernelGGL((k_panel_gemm<SK, false>), dim3(grid), dim3(256), 0, st, m, wd, k, A, lda, B, ldb, P,
-                       (int)nunits, rtiles, ntiles);
+  if (skip >= 0) return hipErrorInvalidValue;
+  // groups or sub-blocks that start or end off a multiple of 4 columns: one workgroup per resident
+  // slot (occupancy is a property of the kernel, cached per process; concurrent first calls compute
+  // the same value)
+  constexpr int SK = 32;
+  const long nunits = (long)ntiles * ((k + CDCLQ_KC - 1) / CDCLQ_KC) * ((wd + PC - 1) / PC);
+  if (nunits > INT32_MAX) return hipErrorInvalidValue;
+  static std::atomic<int> slots{0};
+  if (slots.load(std::memory_order_relaxed) == 0) {
+    int cus = 0, per = 0;
+    hipError_t err = device_cus(&cus);
+    if (err == hipSuccess) err = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_panel_gemm<SK>, 256, 0);
+    if (err != hipSuccess) return err;
+    slots.store(std::max(1, cus * std::max(1, per)), std::memory_order_relaxed);
+  }
+  hipLaunchKernelGGL(k_panel_gemm<SK>, dim3((int)std::min<long>(nunits, slots.load(std::memory_order_relaxed))),
+                     dim3(256), 0, st, m, wd, k, A, lda, B, ldb, P, (int)nunits, rtiles, ntiles);
   return hipGetLastError();
 }
 
@@ -1517,7 +1500,7 @@ hipError_t chain_gemm_mfma(hipStream_t st, int m, int n, int k, float alpha, int
   const long wunits = (long)((m + PR - 1) / PR) * ((n + LPC - 1) / LPC);
   if (beta_one && wunits >= ws && wunits <= INT32_MAX) {
     hipLaunchKernelGGL(k_lazy_wide<true>, dim3(ws), dim3(512), 0, st, m, n, k, A, lda, B, ldb, C, ldc, alpha,
-                       (int)wunits, (float*)nullptr, (const int*)nullptr, kf);
+                       (int)wunits, (float*)nullptr, (const int*)nullptr, kf, -1);
     return hipGetLastError();
   }
   int dslots = 0;
@@ -1526,7 +1509,7 @@ hipError_t chain_gemm_mfma(hipStream_t st, int m, int n, int k, float alpha, int
   const int ntiles = (m + PR - 1) / PR;
   const long nunits = (long)ntiles * ((n + PC - 1) / PC);
   hipLaunchKernelGGL(k_panel_dma<true>, dim3((int)std::min<long>(nunits, dslots)), dim3(256), 0, st, m, n, k, A, lda, B, ldb,
-                     (float*)nullptr, (int)nunits, (const int*)nullptr, ntiles, C, ldc, alpha, beta_one, kf);
+                     (float*)nullptr, (int)nunits, (const int*)nullptr, ntiles, C, ldc, alpha, beta_one, kf, -1);
   return hipGetLastError();
 }
 
@@ -1541,7 +1524,7 @@ hipError_t fold_panels(hipStream_t st, int m, int wd, int np, const float* P, fl
 
 bool refit_folds_chains(int wd) { return wd > 0 && wd <= 128; }  // the matrix-core k_refit_mfma
 
-hipError_t refit_group(hipStream_t st, int rows, int n, int ng, int g, int gi, int rc, const float* G,
+hipError_t refit_group(hipStream_t st, int rows, int n, int ld, int ng, int g, int gi, int rc, const float* G,
                        const float* h32, const uint8_t* codes, float* scales, const float* zeros, float* wq, float* e,
                        const uint8_t* active, double* dlog, uint32_t* dcnt, const float* P, int np) {
   const int wd = std::min(gi * g + g, n) - gi * g;
@@ -1550,21 +1533,21 @@ hipError_t refit_group(hipStream_t st, int rows, int n, int ng, int g, int gi, i
     // the smallest workgroups (shortest chains) whose count still fits two per CU, so that all
     // rows are resident in one round; 64-row ones beyond that
     int cus = 0;
-    const hipError_t err = cu_count(&cus);
+    const hipError_t err = device_cus(&cus);
     if (err != hipSuccess) return err;
     if ((rows + 15) / 16 <= 2 * cus)
-      hipLaunchKernelGGL(k_refit_mfma<16>, dim3((rows + 15) / 16), dim3(256), 0, st, rows, n, ng, g, gi, rc, G, h32,
+      hipLaunchKernelGGL(k_refit_mfma<16>, dim3((rows + 15) / 16), dim3(256), 0, st, rows, n, ld, ng, g, gi, rc, G, h32,
                          codes, scales, zeros, wq, e, active, dlog, dcnt, P, np);
     else if ((rows + 31) / 32 <= 2 * cus)
-      hipLaunchKernelGGL(k_refit_mfma<32>, dim3((rows + 31) / 32), dim3(256), 0, st, rows, n, ng, g, gi, rc, G, h32,
+      hipLaunchKernelGGL(k_refit_mfma<32>, dim3((rows + 31) / 32), dim3(256), 0, st, rows, n, ld, ng, g, gi, rc, G, h32,
                          codes, scales, zeros, wq, e, active, dlog, dcnt, P, np);
     else
-      hipLaunchKernelGGL(k_refit_mfma<64>, dim3((rows + 63) / 64), dim3(256), 0, st, rows, n, ng, g, gi, rc, G, h32,
+      hipLaunchKernelGGL(k_refit_mfma<64>, dim3((rows + 63) / 64), dim3(256), 0, st, rows, n, ld, ng, g, gi, rc, G, h32,
                          codes, scales, zeros, wq, e, active, dlog, dcnt, P, np);
     return hipGetLastError();
   }
 #define REFIT_CASE(N)                                                                                                  \
-  hipLaunchKernelGGL((k_refit<N>), dim3((rows + 3) / 4), dim3(256), 0, st, rows, n, ng, g, gi, rc, G, h32, codes,      \
+  hipLaunchKernelGGL((k_refit<N>), dim3((rows + 3) / 4), dim3(256), 0, st, rows, n, ld, ng, g, gi, rc, G, h32, codes,      \
                      scales, zeros, wq, e, active, dlog, dcnt)
   switch (npl_for(wd)) {
     case 4: REFIT_CASE(4); break;
@@ -1578,7 +1561,7 @@ hipError_t refit_group(hipStream_t st, int rows, int n, int ng, int g, int gi, i
 
 bool cd_folds_chains(int wd) { return wd > 0 && wd <= 1024; }  // the register-resident k_cd<NPL>
 
-hipError_t cd_subblock(hipStream_t st, int rows, int n, int ng, int g, int c0, int wd, int sb, int nsb, int rc,
+hipError_t cd_subblock(hipStream_t st, int rows, int n, int ld, int ng, int g, int c0, int wd, int sb, int nsb, int rc,
                        int sweeps, float* G, const float* h32, const uint8_t* gbits, const float* scales,
                        const float* zeros, uint8_t* codes, float* wq, float* e, const uint8_t* active,
                        const uint8_t* sel, double* dlog, uint32_t* dcnt, int cap, unsigned long long* mid,
@@ -1586,12 +1569,12 @@ hipError_t cd_subblock(hipStream_t st, int rows, int n, int ng, int g, int c0, i
   const dim3 grid((rows + 3) / 4), blk(256);
   if (P && !cd_folds_chains(wd)) return hipErrorInvalidValue;
 #define CD_CASE(N)                                                                                                     \
-  hipLaunchKernelGGL((k_cd<N>), grid, blk, 0, st, rows, n, ng, g, c0, wd, sb, nsb, rc, sweeps, G, h32, gbits, scales,  \
+  hipLaunchKernelGGL((k_cd<N>), grid, blk, 0, st, rows, n, ld, ng, g, c0, wd, sb, nsb, rc, sweeps, G, h32, gbits, scales,  \
                      zeros, codes, wq, e, active, sel, dlog, dcnt, cap, mid, evals, P, np)
   switch (npl_for(wd)) {
     case 1:
       if (P && np > 16)  // many panels: fewer, wider fold batches
-        hipLaunchKernelGGL((k_cd<1, 32>), grid, blk, 0, st, rows, n, ng, g, c0, wd, sb, nsb, rc, sweeps, G, h32, gbits,
+        hipLaunchKernelGGL((k_cd<1, 32>), grid, blk, 0, st, rows, n, ld, ng, g, c0, wd, sb, nsb, rc, sweeps, G, h32, gbits,
                            scales, zeros, codes, wq, e, active, sel, dlog, dcnt, cap, mid, evals, P, np);
       else
         CD_CASE(1);
@@ -1601,7 +1584,7 @@ hipError_t cd_subblock(hipStream_t st, int rows, int n, int ng, int g, int c0, i
     case 8: CD_CASE(8); break;
     case 16: CD_CASE(16); break;
     default:  // wider than 1024 columns: gradient row and column state in memory
-      hipLaunchKernelGGL(k_cd_mem, grid, blk, 0, st, rows, n, ng, g, c0, wd, sb, nsb, rc, sweeps, G,
+      hipLaunchKernelGGL(k_cd_mem, grid, blk, 0, st, rows, n, ld, ng, g, c0, wd, sb, nsb, rc, sweeps, G,
                          h32, gbits, scales, zeros, codes, wq, e, active, sel, dlog, dcnt, cap, mid, evals);
       break;
   }

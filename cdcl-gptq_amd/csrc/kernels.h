@@ -80,8 +80,9 @@ constexpr size_t kGramScratchBytes = 512 + kGramScratchTiles * 16;
 hipError_t gram_scratch(int device, void** ptr);
 
 // ---- k_factor.hip: damping, Cholesky, triangular inverse, U
-hipError_t build_flipped(hipStream_t st, int n, const float* h, const uint32_t* perm, double damp_val, double* a,
-                         float* h32);
+// h32 has rows of ld floats and ld rows (ld >= n), zero past n
+hipError_t build_flipped(hipStream_t st, int n, int ld, const float* h, const uint32_t* perm, double damp_val,
+                         double* a, float* h32);
 hipError_t build_flipped_f64(hipStream_t st, int n, const double* h, double* a);
 hipError_t chol_diag(hipStream_t st, int n, double* a, int k, int kb, int* status, double* pivot);
 hipError_t chol_panel(hipStream_t st, int n, double* a, int k, int kb, const int* status);
@@ -105,13 +106,22 @@ hipError_t gptq_block(hipStream_t st, int rows, int n, int i1, int cnt, int g, i
 hipError_t colloss(hipStream_t st, int rows, int n, int rc, const float* err, double* out);
 hipError_t sub_f32(hipStream_t st, size_t count, const float* a, const float* b, float* out);
 // ---- k_repair.hip: phase 2
+// The residual E (e) and the damped permuted H (h32) of phase 2 have rows of ld floats, ld = n
+// rounded up to 64 (repair_ld), zero in the columns past n (h32 also in the rows past n): the
+// gradient GEMM's k and its 256-column panels then stay whole and 16-byte aligned for every n.
+inline int repair_ld(int n) { return (n + 63) / 64 * 64; }
+// e = a - b over rows x n, zero in columns n .. ld - 1
+hipError_t residual(hipStream_t st, int rows, int n, int ld, const float* a, const float* b, float* e);
+// compute units of the current device (cached per process)
+hipError_t device_cus(int* out);
 // P[p][r][c] = chain over panel p of A[r][k] B[k][c] (r < m, c < wd)
 size_t panel_partials_elems(int m, int wd, int k);
 // Repair gradient: per-panel chains of G = A B into P (np x m x wd), for the listed 128-row tiles
 // of A (all tiles when rtiles is null), then their ordered fold into G (d_out x wd).
 int panel_row_tile();
+// skip >= 0: that panel is left out, P holding the chains of the others in order.
 hipError_t panel_gemm(hipStream_t st, int m, int wd, int k, const float* A, long lda, const float* B, long ldb,
-                      float* P, const int* rtiles, int ntiles);
+                      float* P, const int* rtiles, int ntiles, int skip = -1);
 hipError_t fold_panels(hipStream_t st, int m, int wd, int np, const float* P, float* G, const int* rtiles,
                        int ntiles);
 // f32 chain GEMM on the matrix cores folding one chain per kfold steps of k straight into C:
@@ -133,7 +143,7 @@ hipError_t transpose_f32(hipStream_t st, int n, const float* src, float* dst);
 // Scale refit of group gi from its gradient: G (rows x wd), or, with P, the np per-panel chains of
 // panel_gemm (P[p][rows][wd]) folded in panel order by the kernel itself (no separate fold
 // launch); refit_folds_chains(wd) says whether that form is available.
-hipError_t refit_group(hipStream_t st, int rows, int n, int ng, int g, int gi, int rc, const float* G,
+hipError_t refit_group(hipStream_t st, int rows, int n, int ld, int ng, int g, int gi, int rc, const float* G,
                        const float* h32, const uint8_t* codes, float* scales, const float* zeros, float* wq, float* e,
                        const uint8_t* active, double* dlog, uint32_t* dcnt, const float* P = nullptr, int np = 0);
 bool refit_folds_chains(int wd);
@@ -141,11 +151,49 @@ bool refit_folds_chains(int wd);
 // the np per-panel chains of panel_gemm (P[p][rows][wd]), folded in panel order by the kernel
 // itself (no separate fold launch); cd_folds_chains(wd) says whether that form is available.
 bool cd_folds_chains(int wd);
-hipError_t cd_subblock(hipStream_t st, int rows, int n, int ng, int g, int c0, int wd, int sb, int nsb, int rc,
+hipError_t cd_subblock(hipStream_t st, int rows, int n, int ld, int ng, int g, int c0, int wd, int sb, int nsb, int rc,
                        int sweeps, float* G, const float* h32, const uint8_t* gbits, const float* scales,
                        const float* zeros, uint8_t* codes, float* wq, float* e, const uint8_t* active,
                        const uint8_t* sel, double* dlog, uint32_t* dcnt, int cap, unsigned long long* mid,
                        uint32_t* evals, const float* P = nullptr, int np = 0);
+// ---- k_panel.hip: the refit groups / the 64-column descent sub-blocks of KC panel q, one after
+// another in one launch. P holds the other np - 1 panels' chains over the panel's wdp columns
+// (panel_gemm with skip = q; unread when np == 1). The _ok tests say
+// which group and sub-block widths it takes (else one refit_group / cd_subblock per step).
+struct RefitPanelArgs {
+  int rows, n, ld, ng, g, q, rc, np, wdp;
+  const float* P;
+  const float* h32;
+  const uint8_t* codes;
+  float* scales;
+  const float* zeros;
+  float* wq;
+  float* e;
+  const uint8_t* active;
+  double* dlog;    // [group][rows]
+  uint32_t* dcnt;  // [group][rows]
+};
+struct CdPanelArgs {
+  int rows, n, ld, ng, g, q, nsb, rc, sweeps, cap, np, wdp;
+  const float* P;
+  const float* h32;
+  const uint8_t* gbits;
+  const float* scales;
+  const float* zeros;
+  uint8_t* codes;
+  float* wq;
+  float* e;
+  const uint8_t* active;
+  const uint8_t* sel;  // [chunk][nsb]
+  double* dlog;        // [sub-block][rows][cap]
+  uint32_t* dcnt;      // [sub-block][rows], zeroed by the caller: rows that are not visited keep it
+  unsigned long long* mid;
+  uint32_t* evals;
+};
+bool refit_panel_ok(int n, int g);
+bool cd_panel_ok(int n, int sbw);
+hipError_t refit_panel(hipStream_t st, const RefitPanelArgs& a);
+hipError_t cd_panel(hipStream_t st, const CdPanelArgs& a);
 // Folds one pass's logged deltas into the per-chunk loss (exact reference order); nref refit
 // steps (rlog/rcnt: [nref][rows]) then ncd CD steps (clog: [ncd][rows][cap], ccnt: [ncd][rows]).
 hipError_t pass_accum(hipStream_t st, int rows, int rc, int nchunks, int nref, const double* rlog,

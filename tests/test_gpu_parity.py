@@ -400,6 +400,25 @@ def test_quantize_wide_gradient_tiles(ctx):
                 label="wide gradient tiles")
 
 
+@pytest.mark.parametrize("d_out,n,group", [
+    (33, 40, 0), (70, 100, 0),                       # one group, one panel
+    (40, 300, 8), (1025, 257, 16), (65, 511, 32),    # several groups per 64-column piece, ragged panels
+    (1100, 333, 128), (2049, 520, 32), (2060, 772, 128), (4100, 300, 64),
+    (37, 2600, 64), (19, 4700, 128), (19, 4612, 32),  # 11 and 19 panels: wider chain batches
+])
+def test_quantize_panel_sweeps(ctx, d_out, n, group):
+    """The sweeps that run one KC panel of refit groups or descent sub-blocks per launch: 4, 8 and 16
+    rows per workgroup (at most 1024, at most 2048 and more rows on a 256-CU part) with a ragged last
+    one, groups inside a 64-column piece of H and of two pieces, last panels, pieces and groups of
+    any width, odd n, half of the sub-blocks selected, chunk borders inside a workgroup."""
+    w, x, h, _ = synth_layer(81 + d_out % 13, d_out, n, n + 200)
+    kw = dict(bits=3, group=group, block=128 if group else n, act_order=True, passes=3)
+    assert_same(*run_both(ctx, w, h, row_chunk=37, **kw), label=f"panel sweeps {d_out}x{n} g{group}")
+    if n < 1000:
+        assert_same(*run_both(ctx, w, h, row_chunk=64, refine_frac=0.5, cd_sweeps=2, **kw),
+                    label=f"panel sweeps {d_out}x{n} g{group}, half selected")
+
+
 def test_quantize_descent_fold_of_many_panels(ctx):
     """Gradients of more than 16 KC panels (n = 4608: 18 panels) take the descent form that folds
     the per-panel chains 32 at a time; 2 passes, act-order, against the live oracle."""
