@@ -105,6 +105,21 @@ inline int ensure(cdclq_ctx* ctx, DevBuf& b, size_t bytes) {
   return CDCLQ_OK;
 }
 
+// Pinned host staging of at least `bytes` (kept by the context; a larger request replaces it
+// after the stream has drained, since earlier copies may still read it).
+inline int ensure_pinned(cdclq_ctx* ctx, size_t bytes) {
+  if (ctx->pin_size >= bytes) return CDCLQ_OK;
+  if (ctx->pin) {
+    HIPCK(hipStreamSynchronize(ctx->st));
+    HIPCK(hipHostFree(ctx->pin));
+    ctx->pin = nullptr;
+    ctx->pin_size = 0;
+  }
+  HIPCK(hipHostMalloc(&ctx->pin, bytes, hipHostMallocDefault));
+  ctx->pin_size = bytes;
+  return CDCLQ_OK;
+}
+
 template <class T>
 inline T* P(DevBuf& b) {
   return static_cast<T*>(b.p);

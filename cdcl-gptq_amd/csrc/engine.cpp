@@ -198,21 +198,6 @@ int factor(cdclq_ctx* ctx, int n, double* a, double* y, float* u) {
   return CDCLQ_OK;
 }
 
-// Pinned host staging of at least `bytes` (kept by the context; a larger request replaces it
-// after the stream has drained, since earlier copies may still read it).
-int ensure_pinned(cdclq_ctx* ctx, size_t bytes) {
-  if (ctx->pin_size >= bytes) return CDCLQ_OK;
-  if (ctx->pin) {
-    HIPCK(hipStreamSynchronize(ctx->st));
-    HIPCK(hipHostFree(ctx->pin));
-    ctx->pin = nullptr;
-    ctx->pin_size = 0;
-  }
-  HIPCK(hipHostMalloc(&ctx->pin, bytes, hipHostMallocDefault));
-  ctx->pin_size = bytes;
-  return CDCLQ_OK;
-}
-
 // The G = E H[:, c0:c0+wd] GEMM of phase 2 (src/engine.rs:548, :608): per-panel chains into
 // ctx->part, then folded in panel order into ctx->G.
 int grad_gemm(cdclq_ctx* ctx, int rows, int n, int c0, int wd, const float* e, const float* h32, const int* rtiles,
@@ -1154,25 +1139,12 @@ int cdclq_proxy_loss(cdclq_ctx* ctx, const float* w_t, const float* w_hat, size_
   HIPCK(hipSetDevice(ctx->device));
   const size_t wn = rows * n;
   CK(ensure(ctx, ctx->w_in, wn * 4));
-  CK(ensure(ctx, ctx->t1, wn * 4));
   CK(ensure(ctx, ctx->t2, wn * 4));
   CK(ensure(ctx, ctx->h_in, n * n * 4));
   HIPCK(hipMemcpyAsync(ctx->w_in.p, w_t, wn * 4, hipMemcpyHostToDevice, ctx->st));
   HIPCK(hipMemcpyAsync(ctx->t2.p, w_hat, wn * 4, hipMemcpyHostToDevice, ctx->st));
   HIPCK(hipMemcpyAsync(ctx->h_in.p, h, n * n * 4, hipMemcpyHostToDevice, ctx->st));
-  HIPCK(sub_f32(ctx->st, wn, P<float>(ctx->w_in), P<float>(ctx->t2), P<float>(ctx->t1)));  // e
-  HIPCK(gemm_chain<float>(ctx->st, (int)rows, (int)n, (int)n, 1.0f, 0, P<float>(ctx->t1), (long)n, 1,
-                          P<float>(ctx->h_in), (long)n, 1, P<float>(ctx->t2), (long)n, 1, false, nullptr));
-  const int nb = 1024;
-  CK(ensure(ctx, ctx->proxy_p, nb * 8));
-  HIPCK(proxy_reduce(ctx->st, wn, P<float>(ctx->t1), P<float>(ctx->t2), P<double>(ctx->proxy_p), nb));
-  std::vector<double> part(nb);
-  HIPCK(hipMemcpyAsync(part.data(), ctx->proxy_p.p, nb * 8, hipMemcpyDeviceToHost, ctx->st));
-  HIPCK(hipStreamSynchronize(ctx->st));
-  double s = 0.0;
-  for (double v : part) s += v;
-  *out = s;
-  return CDCLQ_OK;
+  return cdclq_proxy_loss_device(ctx, P<float>(ctx->w_in), P<float>(ctx->t2), rows, n, P<float>(ctx->h_in), out);
 }
 
 int cdclq_device_alloc(cdclq_ctx* ctx, size_t bytes, void** ptr) {

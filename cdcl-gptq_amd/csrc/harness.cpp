@@ -201,28 +201,40 @@ int actgen_sample(cdclq_ctx* ctx, ActGen& g, Rng& rng, size_t tokens, float* x) 
   return CDCLQ_OK;
 }
 
+// A dense rows x n operand of the evaluation's tiles: itself, or a copy in `buf` with rows padded to
+// a multiple of 64 floats (*ld the row stride).
+int eval_operand(cdclq_ctx* ctx, DevBuf& buf, const float* src, size_t rows, size_t n, bool direct, const float** out,
+                 long* ld) {
+  *out = src;
+  *ld = (long)n;
+  if (direct) return CDCLQ_OK;
+  *ld = repair_ld((int)n);
+  CK(ensure(ctx, buf, rows * (size_t)*ld * 4));
+  HIPCK(pad_rows(ctx->st, (long)rows, (int)n, (long)rows, (int)*ld, src, P<float>(buf)));
+  *out = P<float>(buf);
+  return CDCLQ_OK;
+}
+
 int rel_err_device(cdclq_ctx* ctx, const float* w, const float* wq, const float* x, const float* xt, size_t rows,
                    size_t n, size_t t, double* out) {
-  Dev o1, o2, part;
-  const int nb = 1024;
-  HIPCK(o1.alloc(rows * t * 4));
-  HIPCK(o2.alloc(rows * t * 4));
-  HIPCK(part.alloc(2 * nb * 8));
-  // o = W x^T (rows x t): B[k][j] = x[j][k]
-  HIPCK(gemm_chain<float>(ctx->st, (int)rows, (int)t, (int)n, 1.0f, 0, w, (long)n, 1, x, 1, (long)n, o1.as<float>(),
-                          (long)t, 1, false, nullptr));
-  HIPCK(gemm_chain<float>(ctx->st, (int)rows, (int)t, (int)n, 1.0f, 0, wq, (long)n, 1, xt, 1, (long)n, o2.as<float>(),
-                          (long)t, 1, false, nullptr));
-  HIPCK(err_reduce(ctx->st, rows * t, o1.as<float>(), o2.as<float>(), part.as<double>(), nb));
-  std::vector<double> h(2 * nb);
-  HIPCK(hipMemcpyAsync(h.data(), part.p, h.size() * 8, hipMemcpyDeviceToHost, ctx->st));
+  // o = W x^T (rows x t): the four operands share one k, so they are padded together or not at all
+  const bool direct = eval_operand_ok(n, w) && eval_operand_ok(n, wq) && eval_operand_ok(n, x) && eval_operand_ok(n, xt);
+  const float *pw, *pq, *px, *pt;
+  long ld;
+  CK(eval_operand(ctx, ctx->t1, w, rows, n, direct, &pw, &ld));
+  CK(eval_operand(ctx, ctx->t2, wq, rows, n, direct, &pq, &ld));
+  CK(eval_operand(ctx, ctx->x_in, x, t, n, direct, &px, &ld));
+  if (xt == x)
+    pt = px;
+  else
+    CK(eval_operand(ctx, ctx->y_in, xt, t, n, direct, &pt, &ld));
+  CK(ensure(ctx, ctx->proxy_p, eval_partials(rows, t) * 8));
+  CK(ensure_pinned(ctx, 16));
+  double* sums = static_cast<double*>(ctx->pin);
+  HIPCK(rel_err_sums(ctx->st, (int)rows, (int)t, (int)(direct ? n : (n + 31) & ~(size_t)31), pw, pq, ld, px, pt, ld,
+                     P<double>(ctx->proxy_p), sums));
   HIPCK(hipStreamSynchronize(ctx->st));
-  double num = 0.0, den = 0.0;
-  for (int b = 0; b < nb; ++b) {
-    num += h[2 * b];
-    den += h[2 * b + 1];
-  }
-  *out = num / den;
+  *out = sums[0] / sums[1];
   return CDCLQ_OK;
 }
 
@@ -312,22 +324,22 @@ int cdclq_proxy_loss_device(cdclq_ctx* ctx, const float* w_t, const float* w_hat
   *out = 0.0;
   if (rows == 0 || n == 0) return CDCLQ_OK;
   HIPCK(hipSetDevice(ctx->device));
-  const size_t wn = rows * n;
-  Dev e, eh, part;
-  const int nb = 1024;
-  HIPCK(e.alloc(wn * 4));
-  HIPCK(eh.alloc(wn * 4));
-  HIPCK(part.alloc(nb * 8));
-  HIPCK(sub_f32(ctx->st, wn, w_t, w_hat, e.as<float>()));
-  HIPCK(gemm_chain<float>(ctx->st, (int)rows, (int)n, (int)n, 1.0f, 0, e.as<float>(), (long)n, 1, h, (long)n, 1,
-                          eh.as<float>(), (long)n, 1, false, nullptr));
-  HIPCK(proxy_reduce(ctx->st, wn, e.as<float>(), eh.as<float>(), part.as<double>(), nb));
-  std::vector<double> p(nb);
-  HIPCK(hipMemcpyAsync(p.data(), part.p, nb * 8, hipMemcpyDeviceToHost, ctx->st));
+  const bool direct = eval_operand_ok(n, h);
+  const long ld = direct ? (long)n : repair_ld((int)n);
+  CK(ensure(ctx, ctx->t1, rows * (size_t)ld * 4));
+  HIPCK(residual(ctx->st, (int)rows, (int)n, (int)ld, w_t, w_hat, P<float>(ctx->t1)));
+  if (!direct) {  // H with rows (and as many of them as the padded k) of ld floats, zero past n
+    CK(ensure(ctx, ctx->mp, (size_t)ld * ld * 4));
+    HIPCK(pad_rows(ctx->st, (long)n, (int)n, ld, (int)ld, h, P<float>(ctx->mp)));
+    h = P<float>(ctx->mp);
+  }
+  CK(ensure(ctx, ctx->proxy_p, eval_partials(rows, (size_t)ld) * 8));
+  CK(ensure_pinned(ctx, 16));
+  double* sums = static_cast<double*>(ctx->pin);
+  HIPCK(proxy_sum(ctx->st, (int)rows, (int)ld, (int)(direct ? n : (n + 31) & ~(size_t)31), P<float>(ctx->t1), ld, h,
+                  ld, P<double>(ctx->proxy_p), sums));
   HIPCK(hipStreamSynchronize(ctx->st));
-  double s = 0.0;
-  for (double v : p) s += v;
-  *out = s;
+  *out = sums[0];
   return CDCLQ_OK;
 }
 

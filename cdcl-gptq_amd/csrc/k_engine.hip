@@ -568,17 +568,12 @@ __global__ __launch_bounds__(256) void k_colloss(int rows, int n, int rc, const 
 // e = a - b (rows x n), rows of ld floats zero past column n
 __global__ __launch_bounds__(256) void k_residual(int rows, int n, int ld, const float* __restrict__ a,
                                                   const float* __restrict__ b, float* __restrict__ e) {
-  const long idx = (long)blockIdx.x * 256 + threadIdx.x;
-  if (idx >= (long)rows * ld) return;
-  const int r = (int)(idx / ld), c = (int)(idx % ld);
-  const long o = (long)r * n + c;
-  e[idx] = c < n ? a[o] - b[o] : 0.0f;
-}
-
-__global__ __launch_bounds__(256) void k_sub(long count, const float* __restrict__ a, const float* __restrict__ b,
-                                             float* __restrict__ o) {
-  const long idx = (long)blockIdx.x * 256 + threadIdx.x;
-  if (idx < count) o[idx] = a[idx] - b[idx];
+  const long count = (long)rows * ld;
+  for (long idx = (long)blockIdx.x * 256 + threadIdx.x; idx < count; idx += (long)gridDim.x * 256) {
+    const int r = (int)(idx / ld), c = (int)(idx % ld);
+    const long o = (long)r * n + c;
+    e[idx] = c < n ? a[o] - b[o] : 0.0f;
+  }
 }
 
 // Per-chunk loss bookkeeping of one pass, in the reference's order (src/engine.rs:583, :640):
@@ -750,22 +745,6 @@ __global__ __launch_bounds__(256) void k_f64_to_f32(long count, const double* __
     b[idx] = (float)a[idx];
 }
 
-// Block partial sums of (f64)e * (f64)eh for proxy_loss (src/engine.rs:814).
-__global__ __launch_bounds__(256) void k_proxy_reduce(long count, const float* __restrict__ e,
-                                                      const float* __restrict__ eh, double* __restrict__ partial) {
-  __shared__ double red[256];
-  double s = 0.0;
-  for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < count; i += (long)gridDim.x * 256)
-    s += (double)e[i] * (double)eh[i];
-  red[threadIdx.x] = s;
-  __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
-    if (threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) partial[blockIdx.x] = red[0];
-}
-
 }  // namespace
 
 hipError_t diag_extract(hipStream_t st, int n, const float* h, float* diag) {
@@ -848,12 +827,7 @@ hipError_t colloss(hipStream_t st, int rows, int n, int rc, const float* err, do
 }
 
 hipError_t residual(hipStream_t st, int rows, int n, int ld, const float* a, const float* b, float* e) {
-  hipLaunchKernelGGL(k_residual, dim3(nblk((long)rows * ld)), dim3(256), 0, st, rows, n, ld, a, b, e);
-  return hipGetLastError();
-}
-
-hipError_t sub_f32(hipStream_t st, size_t count, const float* a, const float* b, float* out) {
-  hipLaunchKernelGGL(k_sub, dim3(nblk((long)count)), dim3(256), 0, st, (long)count, a, b, out);
+  hipLaunchKernelGGL(k_residual, dim3(gs_blocks((long)rows * ld)), dim3(256), 0, st, rows, n, ld, a, b, e);
   return hipGetLastError();
 }
 
@@ -889,11 +863,6 @@ hipError_t synth_perturb(hipStream_t st, uint64_t seed, uint64_t offset, size_t 
 hipError_t f64_to_f32(hipStream_t st, size_t count, const double* a, float* b) {
   if (!count) return hipSuccess;
   hipLaunchKernelGGL(k_f64_to_f32, dim3(gs_blocks((long)count)), dim3(256), 0, st, (long)count, a, b);
-  return hipGetLastError();
-}
-
-hipError_t proxy_reduce(hipStream_t st, size_t count, const float* e, const float* eh, double* partial, int nblocks) {
-  hipLaunchKernelGGL(k_proxy_reduce, dim3(nblocks), dim3(256), 0, st, (long)count, e, eh, partial);
   return hipGetLastError();
 }
 

@@ -78,32 +78,6 @@ __global__ __launch_bounds__(256) void k_rtn(long d_out, int n, int g, int ng, i
   }
 }
 
-// bench::rel_err's sums (src/bench.rs:114-119): per-block f64 partials of (o1 - o2)^2 and o1^2.
-__global__ __launch_bounds__(256) void k_err_reduce(long count, const float* __restrict__ o1,
-                                                    const float* __restrict__ o2, double* __restrict__ partial) {
-  __shared__ double rn[256], rd[256];
-  double num = 0.0, den = 0.0;
-  for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < count; i += (long)gridDim.x * 256) {
-    const double d = (double)(o1[i] - o2[i]);
-    num += d * d;
-    den += (double)o1[i] * (double)o1[i];
-  }
-  rn[threadIdx.x] = num;
-  rd[threadIdx.x] = den;
-  __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
-    if (threadIdx.x < o) {
-      rn[threadIdx.x] += rn[threadIdx.x + o];
-      rd[threadIdx.x] += rd[threadIdx.x + o];
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) {
-    partial[2 * blockIdx.x] = rn[0];
-    partial[2 * blockIdx.x + 1] = rd[0];
-  }
-}
-
 // ActGen::sample's per-token step (src/bench.rs:71-78): x = (x + noise) * scale[j] * massive[t],
 // with noise = 0.3 * normal drawn on the host in the reference's order.
 __global__ __launch_bounds__(256) void k_act_scale(long tokens, int n, const float* __restrict__ noise,
@@ -149,11 +123,6 @@ hipError_t rtn_rows(hipStream_t st, long d_out, int n, int g, int bits, int mse,
   const long waves = d_out * ng;
   if (waves <= 0) return hipSuccess;
   hipLaunchKernelGGL(k_rtn, dim3(blocks_for(waves * 64)), dim3(256), 0, st, d_out, n, g, ng, bits, mse, w, out);
-  return hipGetLastError();
-}
-
-hipError_t err_reduce(hipStream_t st, size_t count, const float* o1, const float* o2, double* partial, int nblocks) {
-  hipLaunchKernelGGL(k_err_reduce, dim3(nblocks), dim3(256), 0, st, (long)count, o1, o2, partial);
   return hipGetLastError();
 }
 

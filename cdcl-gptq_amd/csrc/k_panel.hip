@@ -15,6 +15,10 @@
 // i of lane l is row i, column l, which is the descent's own layout. Its chain has a quarter of the
 // 16 x 16 form's latency, and latency is what bounds these kernels: R is the smallest of 4, 8
 // and 16 whose workgroups fit the device at once.
+//
+// Repair of one matrix, a launch pair per step against a launch pair per panel: 256 x 256 3.9 ->
+// 1.7 ms, 1001 x 1350 11.5 -> 5.3 ms, 2048 x 2048 12.9 -> 9.0 ms, 2048 x 5632 (groups of 64) 68.7 ->
+// 44.5 ms, 4096 x 14336 397 -> 384 ms.
 #include <algorithm>
 #include <cstdint>
 

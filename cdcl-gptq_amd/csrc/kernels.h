@@ -104,7 +104,6 @@ hipError_t gptq_block(hipStream_t st, int rows, int n, int i1, int cnt, int g, i
                       const float* invd, const uint8_t* gbits, int mse, float* scales, float* zeros, uint8_t* codes,
                       float* wq, float* err, unsigned long long* mid, bool groups_in_block);
 hipError_t colloss(hipStream_t st, int rows, int n, int rc, const float* err, double* out);
-hipError_t sub_f32(hipStream_t st, size_t count, const float* a, const float* b, float* out);
 // ---- k_repair.hip: phase 2
 // The residual E (e) and the damped permuted H (h32) of phase 2 have rows of ld floats, ld = n
 // rounded up to 64 (repair_ld), zero in the columns past n (h32 also in the rows past n): the
@@ -139,6 +138,19 @@ bool chain_gemm_tiles_ok(int m, int n, int k, const float* A, long lda, const fl
                          long ldc);
 hipError_t chain_gemm_tiles(hipStream_t st, int m, int n, int k, const float* A, long lda, const float* B, long ldb,
                             float* C, long ldc, int tri);
+// The evaluation's f64 sums on the same tiles; out[0..1] (device-visible) receives the totals, partial
+// holds eval_partials(m, n) doubles. k % 32 == 0, operands 16-byte aligned with strides that are a
+// multiple of 4 (eval_operand_ok for a dense matrix of n columns; otherwise pad_rows).
+size_t eval_partials(size_t m, size_t n);
+bool eval_operand_ok(size_t n, const float* p);
+// rows x n (dense) copied into rows_out rows of ld floats, zero in the rest
+hipError_t pad_rows(hipStream_t st, long rows, int n, long rows_out, int ld, const float* src, float* dst);
+// sums of (o1 - o2)^2 and o1^2 over o1 = W X^T, o2 = W_hat Xt^T (W, W_hat m x k; X, Xt n x k)
+hipError_t rel_err_sums(hipStream_t st, int m, int n, int k, const float* W, const float* W_hat, long ldw,
+                        const float* X, const float* Xt, long ldx, double* partial, double* out);
+// sum over m x n of e (E H) (E m x k, H k x n); out[1] = 0
+hipError_t proxy_sum(hipStream_t st, int m, int n, int k, const float* E, long lde, const float* H, long ldh,
+                     double* partial, double* out);
 hipError_t transpose_f32(hipStream_t st, int n, const float* src, float* dst);
 // Scale refit of group gi from its gradient: G (rows x wd), or, with P, the np per-panel chains of
 // panel_gemm (P[p][rows][wd]) folded in panel order by the kernel itself (no separate fold
@@ -223,8 +235,6 @@ hipError_t dequant_rows(hipStream_t st, bool packed, int dtype, long d_out, int 
 // ---- k_eval.hip: benchmark-harness evaluation
 // out (d_out x n) = engine::rtn_layer of w with group g
 hipError_t rtn_rows(hipStream_t st, long d_out, int n, int g, int bits, int mse, const float* w, float* out);
-// partial[2b] = sum (o1 - o2)^2, partial[2b+1] = sum o1^2 over block b's share (f64)
-hipError_t err_reduce(hipStream_t st, size_t count, const float* o1, const float* o2, double* partial, int nblocks);
 // x = (x + noise) * scale[j] * massive[t]
 hipError_t act_scale(hipStream_t st, long tokens, int n, const float* noise, const float* scale, const float* massive,
                      float* x);
@@ -250,6 +260,5 @@ hipError_t synth_tokens(hipStream_t st, uint64_t seed, uint64_t row0, size_t t, 
 hipError_t synth_perturb(hipStream_t st, uint64_t seed, uint64_t offset, size_t count, float sigma, const float* x,
                          float* out);
 hipError_t f64_to_f32(hipStream_t st, size_t count, const double* a, float* b);
-hipError_t proxy_reduce(hipStream_t st, size_t count, const float* e, const float* eh, double* partial, int nblocks);
 
 }  // namespace cdclq

@@ -71,6 +71,28 @@ def test_rel_err_and_proxy_loss_match_oracle(ctx):
         a.free()
 
 
+@pytest.mark.parametrize("rows,n,t", [(1, 5, 3), (129, 31, 127), (130, 333, 129), (257, 512, 1100), (3, 1312, 64)])
+def test_rel_err_and_proxy_loss_tile_edges(ctx, rows, n, t):
+    """Sizes around the 128 x 128 tiles and the 32-column stages, dense (n % 32 == 0) and padded
+    operands, one and several KC panels. The products are the oracle's f32 chains bit for bit; only
+    the f64 sums run in another order. A sum of N terms of one sign is off by at most N 2^-53
+    relative in any order, so rel_err's quotient of two such sums, on two sides, by 4 N 2^-53 with
+    N = rows * t; the proxy loss's terms e (e H) cancel, so its bound is 2 N 2^-53 of their absolute
+    sum, N = rows * n."""
+    rng = np.random.default_rng(rows * 7 + n)
+    w = rng.standard_normal((rows, n)).astype(np.float32)
+    wq = (w + 0.01 * rng.standard_normal((rows, n))).astype(np.float32)
+    x = rng.standard_normal((t, n)).astype(np.float32)
+    xt = (x + 0.05 * rng.standard_normal((t, n))).astype(np.float32)
+    for a, b in ((x, x), (x, xt)):
+        g, o = cdclq.rel_err(ctx, w, wq, a, b), O.rel_err(w, wq, a, b, rows, n, t)
+        assert abs(g - o) <= 4 * rows * t * 2.0 ** -53 * abs(o), (g, o)
+    h = (x.T @ x).astype(np.float32)
+    e = (w - wq).astype(np.float64)
+    bound = 2 * 2.0 ** -53 * rows * n * float((np.abs(e) @ np.abs(h.astype(np.float64)) * np.abs(e)).sum())
+    assert abs(cdclq.proxy_loss(w, wq, rows, n, h, ctx) - O.proxy_loss(w, wq, h)) <= bound
+
+
 def test_bench_run_reproduces_the_readme_table(ctx):
     """`cdclq bench --rows 512 --cols 2048 --tokens 16384 --test-tokens 4096` (3 bit, group 128):
     every held-out error and percentage the README prints (README.md:207-219)."""
