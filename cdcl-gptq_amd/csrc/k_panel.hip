@@ -8,17 +8,19 @@
 // E that the previous step left and folding it into its place. Per panel that is two launches
 // instead of two per step, and a GEMM of 256 columns instead of 64 or 128.
 //
-// A workgroup takes R rows, one wavefront per row, and keeps the rows' E over the panel in LDS.
-// The columns of H that a step needs (256 x 64 floats, 64 KB a piece) are loaded directly to LDS,
-// two pieces at a time. The own chains run on v_mfma_f32_4x4x1_16b_f32 with its 16 blocks side by
-// side: A holds 4 rows of E (the same in every block), lane l supplies B = H[k][l], and D register
-// i of lane l is row i, column l, which is the descent's own layout. Its chain has a quarter of the
-// 16 x 16 form's latency, and latency is what bounds these kernels: R is the smallest of 4, 8
-// and 16 whose workgroups fit the device at once.
+// A workgroup takes R rows, a wavefront per row, and keeps the rows' E over the panel in LDS. The
+// columns of H that a step needs (256 x 64 floats, 64 KB a piece) are loaded directly to LDS, two
+// pieces at a time. Latency bounds these kernels: R is the smallest of 4, 8 and 16 whose workgroups
+// fit the device at once. In cycles, one piece of a descent with 8 rows: the own chains 2600 (64
+// v_mfma_f32_16x16x4_f32 of 32 cycles, four steps of k in ascending order each as in mfma_tile.h, beside the
+// next piece's loads), the fold 250, issuing the next chains' and columns' loads behind the piece's
+// 1300, the visits 700 to 2000 (the row with the most moves), barriers 200. One group of a refit with 8
+// rows: the own chains and U H_CC side by side 6900, the fold 800, the sums 1600, the update 400, the
+// next pieces' loads 3000 from the sums on.
 //
 // Repair of one matrix, a launch pair per step against a launch pair per panel: 256 x 256 3.9 ->
-// 1.7 ms, 1001 x 1350 11.5 -> 5.3 ms, 2048 x 2048 12.9 -> 9.0 ms, 2048 x 5632 (groups of 64) 68.7 ->
-// 44.5 ms, 4096 x 14336 397 -> 384 ms.
+// 1.6 ms, 1001 x 1350 11.5 -> 5.1 ms, 2048 x 2048 12.9 -> 8.2 ms, 2048 x 5632 (groups of 64) 68.7 ->
+// 41.8 ms, 4096 x 14336 397 -> 360 ms.
 #include <algorithm>
 #include <cstdint>
 
@@ -40,29 +42,104 @@ constexpr int ES = KC + 4;         // row stride of the staged E (16-byte aligne
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 // Rows [0, kr) of panel row c0 .. and columns col .. col + 63 of H into the piece at LDS offset
-// `dst`, row-major: load i covers rows 4 i .. 4 i + 3 (lane l: row 4 i + (l >> 4), columns 4 (l & 15)).
-// kr is a multiple of 16 and c0 + kr <= ld, col + 64 <= ld (ld is a multiple of 64).
-template <int R>
+// `dst`: load i covers rows 4 i .. 4 i + 3 (lane l: row 4 i + (l >> 4)). Column c of row k lies at position
+// c ^ 16 (k & 3) (at()), so that the four rows that one MFMA step reads side by side start on
+// different banks. kr is a multiple of 16 and c0 + kr <= ld, col + 64 <= ld (ld is a multiple of 64).
+__device__ __forceinline__ int at(int k, int c) { return k * PW + (c ^ ((k & 3) << 4)); }
+
+template <int W>
 __device__ __forceinline__ void load_piece(const float* __restrict__ h32, int ld, int c0, int kr, int col,
                                            uint32_t dst, int wv, int lane) {
-  const float* src = h32 + (long)(c0 + (lane >> 4)) * ld + col + 4 * (lane & 15);
-  for (int i = wv; i < kr / 4; i += R) dma16_untracked(src + (long)(4 * i) * ld, dst + 1024u * (uint32_t)i);
+  const int q = lane >> 4;
+  const float* src = h32 + (long)(c0 + q) * ld + col + 4 * ((lane & 15) ^ (4 * q));
+  for (int i = wv; i < kr / 4; i += W) dma16_untracked(src + (long)(4 * i) * ld, dst + 1024u * (uint32_t)i);
 }
 
-// kr steps of the chains of 4 rows (a: the lane's row of the A operand, 16-byte aligned) and 64
-// columns (h: the lane's column of a piece).
-__device__ __forceinline__ v4f chain4(const float* a, const float* h, int kr) {
+// kr steps (a multiple of 16) of the chains of 16 rows and 16 columns: a = the lane's first A element
+// (row lane & 15, step lane >> 4, the row's steps following one another), b = its first B element (step
+// lane >> 4 of the piece, column lane & 15 of the 16). Register r of the result is row 4 (lane >> 4) + r,
+// column lane & 15. Every instruction waits for the one before it (32 cycles), so the operands are
+// read eight instructions ahead and the reads issued between the instructions.
+__device__ __forceinline__ v4f chain16(const float* ap, const float* bp, int kr) {
+  // LDS addresses in a register each: the reads' offsets then fit the instructions
+  typedef const __attribute__((address_space(3))) float* lds_t;
+  lds_t a = (lds_t)ap, b = (lds_t)bp;
+  asm volatile("" : "+v"(a), "+v"(b));
   v4f acc = {};
-  for (int k = 0; k < kr; k += 16) {
+  int k = 0;
+  for (; k + 128 <= kr; k += 128) {
+    float x[32], y[32];
 #pragma unroll
-    for (int q = 0; q < 16; q += 4) {
-      const v4f x = *reinterpret_cast<const v4f*>(a + k + q);
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        acc = __builtin_amdgcn_mfma_f32_4x4x1f32(x[j], h[(k + q + j) * PW], acc, 0, 0, 0);
+    for (int u = 0; u < 32; ++u) {
+      x[u] = a[k + 4 * u];
+      y[u] = b[(k + 4 * u) * PW];
     }
+#pragma unroll
+    for (int u = 0; u < 32; ++u) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(x[u], y[u], acc, 0, 0, 0);
+    // (a read brings the operands of two instructions)
+    __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
+#pragma unroll
+    for (int u = 0; u < 12; ++u) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);
+  }
+  for (; k < kr; k += 16) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[k + 4 * u], b[(k + 4 * u) * PW], acc, 0, 0, 0);
   }
   return acc;
+}
+
+// The chains of 4 rows and 64 columns on v_mfma_f32_4x4x1_16b_f32, its 16 blocks side by side: piece =
+// the steps' first row of H (a multiple of 4 of the panel's rows), lane l column l. Register i of the
+// result is row i, column l. a(k) = the lane's A element of step k + (lane >> 2) and row lane & 3; the
+// instruction broadcasts the block of its step to the 16 blocks (cbsz 4, abid the block), so that one
+// register serves 16 steps.
+typedef const __attribute__((address_space(3))) float* lds_f;
+
+struct Cols4 {  // a lane's column of a piece: row k at h[k & 3][(k & ~3) * PW]
+  lds_f h[4];
+  __device__ __forceinline__ Cols4(const float* piece, int lane) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      h[j] = (lds_f)(piece + at(j, lane));
+      asm volatile("" : "+v"(h[j]));
+    }
+  }
+};
+
+#define CHAIN4_STEP(B) \
+  acc = __builtin_amdgcn_mfma_f32_4x4x1f32(x, c.h[(B) & 3][(k + ((B) & ~3)) * PW], acc, 4, B, 0)
+#define CHAIN4_QUAD(B) CHAIN4_STEP(B), CHAIN4_STEP(B + 1), CHAIN4_STEP(B + 2), CHAIN4_STEP(B + 3)
+
+// kr steps (and on to a multiple of 4) of one chain. Groups start at multiples of 16, so the rows read
+// stay inside the piece.
+template <class FA>
+__device__ __forceinline__ void chain4(FA a, const Cols4& c, int kr, v4f& acc) {
+  float x = a(0);
+  int k = 0;
+  for (; k + 16 <= kr; k += 16) {
+    const float xn = a(min(k + 16, (kr - 1) & ~15));
+    CHAIN4_QUAD(0), CHAIN4_QUAD(4), CHAIN4_QUAD(8), CHAIN4_QUAD(12);
+    x = xn;
+  }
+  if (k < kr) CHAIN4_QUAD(0);
+  if (k + 4 < kr) CHAIN4_QUAD(4);
+  if (k + 8 < kr) CHAIN4_QUAD(8);
+  if (k + 12 < kr) CHAIN4_QUAD(12);
+}
+#undef CHAIN4_QUAD
+#undef CHAIN4_STEP
+
+// The loads into v have arrived from here on. The compiler counts the loads it knows of; without this,
+// the wait before their first use would also wait for the direct-to-LDS loads issued since.
+template <int NB>
+__device__ __forceinline__ void arrived(float (&v)[NB]) {
+#pragma unroll
+  for (int u = 0; u < NB; ++u) asm volatile("" : "+v"(v[u]));
 }
 
 // NB of a row's other-panel chains in flight: slots u0 .. u0 + NB - 1 of P (those past nf repeat the
@@ -105,8 +182,11 @@ __device__ __forceinline__ float fold_with_own(const float* __restrict__ src, ui
 // ---- Coordinate descent over the panel's 64-column sub-blocks (src/engine.rs:600-658), decisions
 // and accounting as in k_cd: every lane evaluates its own column with the current gradient, and the
 // lowest column at or after the cursor whose code changes is the next move of the sequential visit.
+// Wavefronts: the first R have a row; 0 to 3 run the own chains while the others (at least four) load
+// the next piece.
 template <int R, int NB>
-__global__ __launch_bounds__(64 * R) void k_cd_panel(CdPanelArgs a) {
+__global__ __launch_bounds__(64 * (R < 8 ? 8 : R)) void k_cd_panel(CdPanelArgs a) {
+  constexpr int W = R < 8 ? 8 : R;
   __shared__ __align__(16) float Hs[2][PIECE];
   __shared__ __align__(16) float Es[R * ES];
   __shared__ float Gs[R * PW];
@@ -115,14 +195,17 @@ __global__ __launch_bounds__(64 * R) void k_cd_panel(CdPanelArgs a) {
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = a.n, ld = a.ld, q = a.q, c0 = q * KC;
   const int kc = min(KC, n - c0), npc = (kc + PW - 1) / PW, kr = (kc + 15) & ~15;
-  const int r = blockIdx.x * R + wv, rr = min(r, a.rows - 1), chunk = rr / a.rc;
+  const bool roww = wv < R;
+  const int wvr = min(wv, R - 1);
+  const int r = blockIdx.x * R + wvr, rr = min(r, a.rows - 1), chunk = rr / a.rc;
   const int sb0 = q * (KC / PW);
   // pieces (= sub-blocks) that this row, and the workgroup, work on
   if (tid == 0) need = 0;
   __syncthreads();
-  uint32_t pick = 0;
-  if (r < a.rows && a.active[chunk])
-    for (int j = 0; j < npc; ++j) pick |= a.sel[(long)chunk * a.nsb + sb0 + j] ? 1u << j : 0u;
+  uint32_t act = a.active[chunk], chosen = a.sel[(long)chunk * a.nsb + sb0 + min(lane, npc - 1)];
+  asm volatile("" : "+v"(act), "+v"(chosen));  // both loads issued before either is tested
+  const uint32_t pick =
+      roww && r < a.rows && __builtin_amdgcn_readfirstlane(act) ? (uint32_t)__ballot(chosen && lane < npc) : 0u;
   if (lane == 0 && pick) atomicOr(&need, pick);
   __syncthreads();
   uint32_t todo = __builtin_amdgcn_readfirstlane(need);
@@ -131,20 +214,13 @@ __global__ __launch_bounds__(64 * R) void k_cd_panel(CdPanelArgs a) {
   const uint32_t hs0 = lds_offset(&Hs[0][0]);
   int j = __builtin_ctz(todo), buf = 0;
   todo &= todo - 1;
-  {
-    v4f ev = {};
-    if (4 * lane < a.wdp) ev = *reinterpret_cast<const v4f*>(a.e + (long)rr * ld + c0 + 4 * lane);
-    load_piece<R>(a.h32, ld, c0, kr, c0 + PW * j, hs0, wv, lane);
-    *reinterpret_cast<v4f*>(&Es[wv * ES + 4 * lane]) = ev;
-  }
-  wait_vmcnt<0>();
   const long pstride = (long)a.rows * a.wdp;
   const int nf = a.np - 1;  // the other panels, slot u of P: panel u + (u >= q)
   const float* prow = a.P + (long)rr * a.wdp;
   float v[NB];
   struct Col {  // a column's state and parameters, one column per lane
-    float wq, sc, zz, mq;
-    int code;
+    float wq, sc, zz;
+    int code, bits;
   };
   auto load_col = [&](int jj) {
     const int wd = min(PW, kc - PW * jj), col = c0 + PW * jj + min(lane, wd - 1), gi = col / a.g;
@@ -153,32 +229,53 @@ __global__ __launch_bounds__(64 * R) void k_cd_panel(CdPanelArgs a) {
     c.code = (int)a.codes[(long)rr * n + col];
     c.sc = a.scales[(long)rr * a.ng + gi];
     c.zz = a.zeros[(long)rr * a.ng + gi];
-    c.mq = (float)((1u << a.gbits[gi]) - 1u);
+    c.bits = a.gbits[gi];
     return c;
   };
-  if (nf > 0) load_chains<NB>(prow + PW * j, lane, pstride, 0, nf, v);
-  Col nxt = load_col(j);
+  Col nxt;
+  {
+    // (the piece first: loads return in order, and it is the largest)
+    load_piece<W>(a.h32, ld, c0, kr, c0 + PW * j, hs0, wv, lane);
+    v4f ev = {};
+    if (4 * lane < a.wdp) ev = *reinterpret_cast<const v4f*>(a.e + (long)rr * ld + c0 + 4 * lane);
+    if (nf > 0) load_chains<NB>(prow + PW * j, lane, pstride, 0, nf, v);
+    nxt = load_col(j);
+    if (roww) *reinterpret_cast<v4f*>(&Es[wv * ES + 4 * lane]) = ev;
+  }
+  wait_vmcnt<0>();
   lds_barrier();
+  // This wavefront's part of the next piece has landed once at most the chains' loads issued after
+  // it are outstanding (a row's; the column's come on top, so this waits for a few of the chains too).
+  auto wait_part = [&]() {
+    if (roww && nf > 0)
+      wait_vmcnt<(NB < 60 ? NB : 60)>();
+    else
+      wait_vmcnt<0>();
+  };
   uint32_t nevals = 0, nnear = 0;
   while (true) {
     const int jn = todo ? __builtin_ctz(todo) : -1;
-    if (jn >= 0) {  // the next piece, into the buffer whose readers passed the last barrier
-      todo &= todo - 1;
-      load_piece<R>(a.h32, ld, c0, kr, c0 + PW * jn, hs0 + (uint32_t)((buf ^ 1) * PIECE * 4), wv, lane);
-    }
-    if (wv < R / 4) {  // the own chains of rows 4 wv .. 4 wv + 3
-      const v4f g = chain4(&Es[(4 * wv + (lane & 3)) * ES], &Hs[buf][lane], kr);
+    if (jn >= 0) todo &= todo - 1;
+    arrived(v);
+    asm volatile("" : "+v"(nxt.wq), "+v"(nxt.sc), "+v"(nxt.zz), "+v"(nxt.bits), "+v"(nxt.code));
+    if (jn >= 0 && wv >= 4)  // the next piece, into the buffer whose readers passed the last barrier
+      load_piece<W - 4>(a.h32, ld, c0, kr, c0 + PW * jn, hs0 + (uint32_t)((buf ^ 1) * PIECE * 4), wv - 4, lane);
+    if (wv < 4) {  // the own chains of columns 16 wv .. + 15
+      const int q4 = lane >> 4, i = lane & 15;
+      const float* ea = &Es[min(i, R - 1) * ES + q4];
+      const float* hb = &Hs[buf][at(q4, 16 * wv + i)];
+      const v4f g = chain16(ea, hb, kr);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) Gs[(4 * wv + i) * PW + lane] = g[i];
+      for (int u = 0; u < 4; ++u) {
+        if (4 * q4 + u < R) Gs[(4 * q4 + u) * PW + 16 * wv + i] = g[u];
+      }
     }
     lds_barrier();
     const int wd = min(PW, kc - PW * j);
     const float* hcc = &Hs[buf][PW * j * PW];  // the sub-block's rows and columns of H
-    float gg = fold_with_own<NB>(prow + PW * j, lane, pstride, q, nf, Gs[wv * PW + lane], v);
+    float gg = fold_with_own<NB>(prow + PW * j, lane, pstride, q, nf, Gs[wvr * PW + lane], v);
     const Col cur = nxt;
-    wait_vmcnt<0>();  // this wave's part of the next piece (everything else has been used)
-    __builtin_amdgcn_sched_barrier(0);
-    if (jn >= 0) {
+    if (jn >= 0 && roww) {
       if (nf > 0) load_chains<NB>(prow + PW * jn, lane, pstride, 0, nf, v);
       nxt = load_col(jn);
     }
@@ -187,7 +284,8 @@ __global__ __launch_bounds__(64 * R) void k_cd_panel(CdPanelArgs a) {
       const uint64_t inmask = __ballot(in);
       float mwq = cur.wq, me = Es[wv * ES + PW * j + lane];
       int mc = cur.code;
-      const float hd = hcc[min(lane, wd - 1) * (PW + 1)], sc = cur.sc, zz = cur.zz, mq = cur.mq;
+      const float hd = hcc[at(min(lane, wd - 1), min(lane, wd - 1))], sc = cur.sc, zz = cur.zz;
+      const float mq = (float)((1u << cur.bits) - 1u);
       const long step = (long)(sb0 + j) * a.rows + r;
       double* dl = a.dlog + step * a.cap;
       uint32_t moves = 0;
@@ -212,7 +310,7 @@ __global__ __launch_bounds__(64 * R) void k_cd_panel(CdPanelArgs a) {
           const float d32 = (2.0f * de) * gj + (de * de) * hjj;
           if (lane == 0) dl[moves] = (double)d32;
           ++moves;
-          gg = gg + de * hcc[jl * PW + lane];  // lanes past wd take values that are never used
+          gg = gg + de * hcc[at(jl, lane)];  // lanes past wd take values that are never used
           if (lane == jl) {
             mwq = newdq;
             mc = qc;
@@ -223,6 +321,7 @@ __global__ __launch_bounds__(64 * R) void k_cd_panel(CdPanelArgs a) {
         }
         if (!changed) break;
       }
+      if (jn >= 0 && wv >= 4) wait_part();
       if (moves && in) {
         const int col = c0 + PW * j + lane;
         a.wq[(long)r * n + col] = mwq;
@@ -233,6 +332,7 @@ __global__ __launch_bounds__(64 * R) void k_cd_panel(CdPanelArgs a) {
       if (lane == 0) a.dcnt[step] = moves;
     }
     if (jn < 0) break;
+    if (wv >= 4 && !((pick >> j) & 1)) wait_part();
     lds_barrier();
     j = jn;
     buf ^= 1;
@@ -253,17 +353,20 @@ __global__ __launch_bounds__(64 * R) void k_cd_panel(CdPanelArgs a) {
 template <int R, int NB, int NH>
 __global__ __launch_bounds__(64 * R) void k_refit_panel(RefitPanelArgs a) {
   constexpr int PS = 64 * NH + 4;              // row stride of the products (16-byte aligned)
-  constexpr int ZN = NH == 2 ? 2 : 32;         // groups of a panel
+  constexpr int ZN = NH == 2 ? 2 : 16;         // groups of a panel
   constexpr int RG = R / 4, NT = RG * NH;      // row quads; chains of each kind
+  // 16 rows of 128-column groups: the products u hu lie in the second piece's buffer; otherwise LDS
+  // has room for them, and both pieces of the next group load as soon as the chains are done
+  constexpr bool PHIN = R == 16 && NH == 2;
   static_assert(2 * NT <= R, "a wavefront per chain");
   __shared__ __align__(16) float Hs[2][PIECE];
   __shared__ __align__(16) float Es[R * ES];
   __shared__ uint32_t Cs[R * KC / 4];          // codes, one byte per column
   __shared__ __align__(16) float PG[R * PS];                 // the own chains, then the products u g
-  __shared__ __align__(16) float PH1[NH == 1 ? R * PS : 1];
+  __shared__ __align__(16) float PH1[PHIN ? 1 : R * PS];
   __shared__ float Zs[R * ZN], snew[R];
   __shared__ int lv[R], mv[R], nlive;
-  float* PH = NH == 2 ? &Hs[1][0] : PH1;       // the products u hu
+  float* PH = PHIN ? &Hs[1][0] : PH1;          // the products u hu
   const int tid = threadIdx.x, lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = a.n, ld = a.ld, q = a.q, g = a.g, ng = a.ng, c0 = q * KC;
@@ -280,21 +383,6 @@ __global__ __launch_bounds__(64 * R) void k_refit_panel(RefitPanelArgs a) {
 
   const uint32_t hs0 = lds_offset(&Hs[0][0]);
   uint8_t* cb = reinterpret_cast<uint8_t*>(Cs) + wv * KC;
-  {
-    v4f ev = {};
-    if (4 * lane < a.wdp) ev = *reinterpret_cast<const v4f*>(a.e + (long)rr * ld + c0 + 4 * lane);
-    uint8_t cv[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) cv[i] = a.codes[(long)rr * n + c0 + min(64 * i + lane, kc - 1)];
-    const float z = a.zeros[(long)rr * ng + g0 + min(lane, gcnt - 1)];
-    load_piece<R>(a.h32, ld, c0, kr, c0, hs0, wv, lane);
-    if (NH == 2 && kc > PW) load_piece<R>(a.h32, ld, c0, kr, c0 + PW, hs0 + PIECE * 4, wv, lane);
-    *reinterpret_cast<v4f*>(&Es[wv * ES + 4 * lane]) = ev;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) cb[64 * i + lane] = cv[i];
-    if (lane < ZN) Zs[wv * ZN + lane] = z;
-  }
-  wait_vmcnt<0>();
   const long pstride = (long)a.rows * a.wdp;
   const int nf = a.np - 1;
   const float* prow = a.P + (long)rr * a.wdp;
@@ -311,7 +399,23 @@ __global__ __launch_bounds__(64 * R) void k_refit_panel(RefitPanelArgs a) {
     }
     if (wv == 0) sold_n = a.scales[(long)min(r0 + min(lane, R - 1), a.rows - 1) * ng + g0 + t];
   };
-  prefetch(0);
+  {
+    // (the pieces first: loads return in order, and they are the largest)
+    load_piece<R>(a.h32, ld, c0, kr, c0, hs0, wv, lane);
+    if (NH == 2 && kc > PW) load_piece<R>(a.h32, ld, c0, kr, c0 + PW, hs0 + PIECE * 4, wv, lane);
+    v4f ev = {};
+    if (4 * lane < a.wdp) ev = *reinterpret_cast<const v4f*>(a.e + (long)rr * ld + c0 + 4 * lane);
+    uint8_t cv[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) cv[i] = a.codes[(long)rr * n + c0 + min(64 * i + lane, kc - 1)];
+    const float z = a.zeros[(long)rr * ng + g0 + min(lane, gcnt - 1)];
+    prefetch(0);
+    *reinterpret_cast<v4f*>(&Es[wv * ES + 4 * lane]) = ev;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) cb[64 * i + lane] = cv[i];
+    if (lane < ZN) Zs[wv * ZN + lane] = z;
+  }
+  wait_vmcnt<0>();
   lds_barrier();
   for (int t = 0; t < gcnt; ++t) {
     const int off = t * g, o = NH == 2 ? 0 : off % PW, wd = min(g, kc - off), gi = g0 + t;
@@ -323,88 +427,95 @@ __global__ __launch_bounds__(64 * R) void k_refit_panel(RefitPanelArgs a) {
     const int tk = wv % NT, rg = tk % RG, h = tk / RG;
     const bool own = wv < NT, hut = wv >= NT && wv < 2 * NT;
     const bool cols = 64 * h < wd;  // (wd <= 64: the second piece is not loaded)
-    v4f ph = {};
-    if (own && cols) {
-      const v4f gv = chain4(&Es[(4 * rg + (lane & 3)) * ES], &Hs[slot + h][lane], kr);
-      const int kcol = 64 * h + lane - o;
-      if (kcol >= 0 && kcol < wd) {
+    const int kcol = 64 * h + lane - o;
+    const uint8_t* cbytes = reinterpret_cast<const uint8_t*>(Cs);
+    v4f gv = {}, hu = {}, ph = {};
+    if (cols && (own || hut)) {
+      const float* ea = &Es[(4 * rg + (lane & 3)) * ES + (lane >> 2)];
+      // hu: one chain of wd <= KC steps (sgemm at src/engine.rs:560); rows of H past n are zero, so a
+      // step past wd (the last group's remainder up to a multiple of 4) adds a zero product
+      const float za = Zs[(4 * rg + (lane & 3)) * ZN + t];
+      const uint8_t* crow = cbytes + (4 * rg + (lane & 3)) * KC + off + (lane >> 2);
+      auto ae = [&](int k) { return ea[k]; };
+      auto au = [&](int k) { return (float)crow[k] - za; };
+      const Cols4 he(&Hs[slot + h][0], lane), hc(&Hs[slot + h][off * PW], lane);
+      if (own)
+        chain4(ae, he, kr, gv);
+      else
+        chain4(au, hc, wd, hu);
+      if (own && kcol >= 0 && kcol < wd) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) PG[(4 * rg + i) * PS + kcol] = gv[i];
       }
-    } else if (hut && cols) {
-      // one chain of wd <= KC steps (sgemm at src/engine.rs:560); rows of H past n are zero, so a
-      // step past wd (the last group's remainder up to a multiple of 4) adds a zero product
-      const float za = Zs[(4 * rg + (lane & 3)) * ZN + t];
-      const uint32_t* crow = Cs + ((4 * rg + (lane & 3)) * KC + off) / 4;
-      const float* hc = &Hs[slot + h][off * PW + lane];
-      v4f acc = {};
-      for (int k = 0; k < wd; k += 4) {
-        const uint32_t w = crow[k >> 2];
+      if (hut) {
 #pragma unroll
-        for (int jj = 0; jj < 4; ++jj)
-          acc = __builtin_amdgcn_mfma_f32_4x4x1f32((float)((w >> (8 * jj)) & 0xffu) - za, hc[(k + jj) * PW], acc, 0,
-                                                   0, 0);
+        for (int i = 0; i < 4; ++i) {  // panel end C = fma(1, chain, 0), then u_k * hu_k
+          const int row = 4 * rg + i;
+          const float u = (float)cbytes[row * KC + min(max(off + kcol, 0), KC - 1)] - Zs[row * ZN + t];
+          ph[i] = u * __builtin_fmaf(1.0f, hu[i], 0.0f);
+        }
       }
-      const int kcol = 64 * h + lane - o;
-      const uint8_t* cbytes = reinterpret_cast<const uint8_t*>(Cs);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {  // panel end C = fma(1, chain, 0), then u_k * hu_k
-        const int row = 4 * rg + i;
-        const float u = (float)cbytes[row * KC + min(max(off + kcol, 0), KC - 1)] - Zs[row * ZN + t];
-        ph[i] = u * __builtin_fmaf(1.0f, acc[i], 0.0f);
-      }
-      if (NH == 1 && kcol >= 0 && kcol < wd) {
+      if (!PHIN && hut && kcol >= 0 && kcol < wd) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) PH[(4 * rg + i) * PS + kcol] = ph[i];
       }
     }
-    lds_barrier();  // the chains are done: both buffers of a 128-column group are free
-    if (NH == 2) {
-      if (more) load_piece<R>(a.h32, ld, c0, kr, c0 + offn, hs0, wv, lane);
-      if (hut && cols) {
-        const int kcol = 64 * h + lane;
-        if (kcol < wd) {
 #pragma unroll
-          for (int i = 0; i < 4; ++i) PH[(4 * rg + i) * PS + kcol] = ph[i];
-        }
-      }
+    for (int hh = 0; hh < NH; ++hh) arrived(v[hh]);
+    arrived(wqn);
+    asm volatile("" : "+v"(sold_n));
+    lds_barrier();  // the chains are done: both buffers of a 128-column group are free
+    if (PHIN && hut && cols && kcol < wd) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) PH[(4 * rg + i) * PS + kcol] = ph[i];
     }
     float wqv[NH], uu[NH];
     const float z = Zs[wv * ZN + t], sold = sold_n;
 #pragma unroll
     for (int hh = 0; hh < NH; ++hh) {
-      const int kcol = 64 * hh + lane - o, kq = min(max(kcol, 0), wd - 1);
+      const int kl = 64 * hh + lane - o, kq = min(max(kl, 0), wd - 1);
       const float gg = fold_with_own<NB>(prow, off + kq, pstride, q, nf, PG[wv * PS + kq], v[hh]);
       uu[hh] = (float)cb[off + kq] - z;
       wqv[hh] = wqn[hh];
-      if (kcol >= 0 && kcol < wd) PG[wv * PS + kcol] = uu[hh] * gg;
+      if (kl >= 0 && kl < wd) PG[wv * PS + kl] = uu[hh] * gg;
     }
     lds_barrier();
-    if (wv == 0 && lane < R) {
-      // num, den: separate multiply and add, sequential in k (src/engine.rs:562-566); then the
-      // closed-form f16 scale and its acceptance test (:567-587)
-      const int row = r0 + lane;
-      const float* pg = PG + lane * PS;
-      const float* ph = PH + lane * PS;
-      float num = 0.0f, den = 0.0f;
+    if (NH == 2 && more && wv > 0) {  // the next group's pieces, while wavefront 0 adds
+      load_piece<R - 1>(a.h32, ld, c0, kr, c0 + offn, hs0, wv - 1, lane);
+      if (!PHIN && offn + PW < kc) load_piece<R - 1>(a.h32, ld, c0, kr, c0 + offn + PW, hs0 + PIECE * 4, wv - 1, lane);
+    }
+    float num = 0.0f, den = 0.0f;
+    if (wv == 0) {
+      // num, den: separate multiply and add, sequential in k (src/engine.rs:562-566), num on lane
+      // `row`, den on lane 32 + row; 16 columns are read while the 16 before them are added
+      const float* ps = (lane < 32 ? PG : PH) + min(lane & 31, R - 1) * PS;
+      v4f x[4], y[4];
+      auto rd = [&](int c, v4f (&v)[4]) {
+#pragma unroll
+        for (int jj = 0; jj < 4; ++jj) v[jj] = *reinterpret_cast<const v4f*>(ps + c + 4 * jj);
+      };
+      auto add = [&](const v4f (&v)[4]) {
+#pragma unroll
+        for (int jj = 0; jj < 16; ++jj) num = num + v[jj >> 2][jj & 3];
+      };
       int k = 0;
-      for (; k + 8 <= wd; k += 8) {
-        v4f x[2], y[2];
-#pragma unroll
-        for (int jj = 0; jj < 2; ++jj) {
-          x[jj] = *reinterpret_cast<const v4f*>(pg + k + 4 * jj);
-          y[jj] = *reinterpret_cast<const v4f*>(ph + k + 4 * jj);
-        }
-#pragma unroll
-        for (int jj = 0; jj < 8; ++jj) {
-          num = num + x[jj >> 2][jj & 3];
-          den = den + y[jj >> 2][jj & 3];
+      if (wd >= 32) {
+        rd(0, x);
+        for (; k + 32 <= wd; k += 32) {
+          rd(k + 16, y);
+          __builtin_amdgcn_sched_barrier(0);
+          add(x);
+          rd(min(k + 32, wd - 16) & ~3, x);  // (after the last pair: read and not used)
+          __builtin_amdgcn_sched_barrier(0);
+          add(y);
         }
       }
-      for (; k < wd; ++k) {
-        num = num + pg[k];
-        den = den + ph[k];
-      }
+      for (; k < wd; ++k) num = num + ps[k];
+      den = __shfl(num, (lane & 31) + 32, 64);
+    }
+    if (wv == 0 && lane < R) {
+      // the closed-form f16 scale and its acceptance test (:567-587)
+      const int row = r0 + lane;
       int moved = 0;
       float s_new = 0.0f;
       if (lv[lane]) {
@@ -424,20 +535,20 @@ __global__ __launch_bounds__(64 * R) void k_refit_panel(RefitPanelArgs a) {
       snew[lane] = s_new;
     }
     if (more) {
-      if (NH == 1) wait_vmcnt<0>();  // the next piece's loads (issued before the chains)
+      if (!PHIN) wait_vmcnt<0>();  // the next pieces' loads, issued at the latest after the chains
       __builtin_amdgcn_sched_barrier(0);
       prefetch(t + 1);
     }
     lds_barrier();
-    if (NH == 2 && more && offn + PW < kc)
+    if (PHIN && more && offn + PW < kc)
       load_piece<R>(a.h32, ld, c0, kr, c0 + offn + PW, hs0 + PIECE * 4, wv, lane);
     if (mv[wv]) {  // e += W_hat - ndq, W_hat = ndq
       const float s_new = snew[wv];
 #pragma unroll
       for (int hh = 0; hh < NH; ++hh) {
-        const int kcol = 64 * hh + lane - o;
-        if (kcol >= 0 && kcol < wd) {
-          const int pc = off + kcol;
+        const int kl = 64 * hh + lane - o;
+        if (kl >= 0 && kl < wd) {
+          const int pc = off + kl;
           const float ndq = s_new * uu[hh];
           const float ne = Es[wv * ES + pc] + (wqv[hh] - ndq);
           Es[wv * ES + pc] = ne;
@@ -447,7 +558,7 @@ __global__ __launch_bounds__(64 * R) void k_refit_panel(RefitPanelArgs a) {
       }
     }
     if (!more) break;
-    if (NH == 2) wait_vmcnt<0>();
+    if (PHIN) wait_vmcnt<0>();
     lds_barrier();
   }
 }
@@ -457,7 +568,7 @@ int panel_rows(int rows, int cus) { return rows <= 4 * cus ? 4 : (rows <= 8 * cu
 
 }  // namespace
 
-bool refit_panel_ok(int n, int g) { return g >= 8 && g <= 128 && (g == 128 || 64 % g == 0 || g >= n); }
+bool refit_panel_ok(int n, int g) { return g <= 128 && (g >= n || g == 128 || (g >= 16 && 64 % g == 0)); }
 bool cd_panel_ok(int n, int sbw) { return sbw == PW || (sbw >= n && n <= PW); }
 
 hipError_t refit_panel(hipStream_t st, const RefitPanelArgs& a) {
@@ -500,7 +611,7 @@ hipError_t cd_panel(hipStream_t st, const CdPanelArgs& a) {
   const hipError_t err = device_cus(&cus);
   if (err != hipSuccess) return err;
   const int R = panel_rows(a.rows, cus);
-  const dim3 grid((a.rows + R - 1) / R), blk(64 * R);
+  const dim3 grid((a.rows + R - 1) / R), blk(64 * std::max(R, 8));
 #define CD_PANEL_R(RR)                                                               \
   do {                                                                               \
     if (a.np <= 9)                                                                   \
