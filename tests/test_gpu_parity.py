@@ -264,6 +264,20 @@ def test_upper_chol_bitexact(ctx, n):
     assert np.array_equal(ug.view(np.uint32), uo.view(np.uint32)), f"{(ug != uo).sum()} U entries differ"
 
 
+@pytest.mark.parametrize("n", [7, 8, 9, 88, 95, 97, 104, 111, 113, 191, 208, 289])
+@pytest.mark.parametrize("sparse", [False, True])
+def test_upper_chol_block_edges_bitexact(ctx, n, sparse):
+    """Blocks of 96 that end inside, at and after 8 columns and 16 rows; block-diagonal matrices give
+    exact zeros, whose signs the inverse's sums decide."""
+    h = rand_spd(n, n + 5)
+    if sparse:
+        i = np.arange(n)
+        h = h * (i[:, None] // 5 == i[None, :] // 5)
+    ug = cdclq.upper_chol_of_inverse(h, n, ctx)
+    uo = O.upper_chol_of_inverse(h)
+    assert np.array_equal(ug.view(np.uint32), uo.view(np.uint32)), f"{(ug != uo).sum()} U entries differ"
+
+
 def _spd_fast(n, seed):
     """M M^T / n + I with M n x (n + 8) from numpy's generator (rand_spd's per-draw loop is slow at
     this size); any SPD input serves for bit parity."""
