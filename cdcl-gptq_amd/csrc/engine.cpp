@@ -735,7 +735,7 @@ int gram_batch_device(cdclq_ctx* ctx, int count, const float* const* xs, const f
   HIPCK(hipMemcpyAsync(flags.data(), status, flags.size() * 4, hipMemcpyDeviceToHost, st));
   HIPCK(hipStreamSynchronize(st));
   // Jobs whose tiles are all interior go to the direct-to-LDS kernel, the rest to k_gram_mfma.
-  std::vector<int4> tiles[2];
+  std::vector<int4> tiles[3];
   for (size_t i = 0; i < jobs.size(); ++i) {
     const bool sym = jobs[i].x == jobs[i].y && flags[4 * i] == 0;
     if (gram_dma_eligible(jobs[i].n, jobs[i].t, jobs[i].x, jobs[i].y))
@@ -745,8 +745,11 @@ int gram_batch_device(cdclq_ctx* ctx, int count, const float* const* xs, const f
   }
   // XCD-aware order: workgroup w runs on XCD w % 8. The direct-to-LDS tiles go in gangs of 4 x 8
   // neighbouring tiles, one gang per XCD at a time (the gang's 32 workgroups share 4 X and 8 Y
-  // stripes in that XCD's L2); the others in a contiguous run per XCD (sharing X stripes).
-  gram_dma_order(tiles[1]);
+  // stripes in that XCD's L2), a short last round in parts; the others in a contiguous run per XCD
+  // (sharing X stripes).
+  int cus = 0;
+  HIPCK(device_cus(&cus));
+  gram_dma_order(cus, tiles[1], tiles[2]);
   {
     auto& tl = tiles[0];
     const size_t nx = 8, m = tl.size();
@@ -760,7 +763,7 @@ int gram_batch_device(cdclq_ctx* ctx, int count, const float* const* xs, const f
       }
     tl.swap(ord);
   }
-  const size_t ntile = tiles[0].size() + tiles[1].size();
+  const size_t ntile = tiles[0].size() + tiles[1].size() + tiles[2].size();
   GramJob* djobs;
   int4* dtiles;
   int* prog = nullptr;  // gang pacing words, one per tile slot (none on the allocation-free path)
@@ -778,13 +781,15 @@ int gram_batch_device(cdclq_ctx* ctx, int count, const float* const* xs, const f
     HIPCK(zero_words(st, prog, (int)ntile));
   }
   HIPCK(hipMemcpyAsync(djobs, jobs.data(), jobs.size() * sizeof(GramJob), hipMemcpyHostToDevice, st));
-  HIPCK(hipMemcpyAsync(dtiles, tiles[0].data(), tiles[0].size() * sizeof(int4), hipMemcpyHostToDevice, st));
-  HIPCK(hipMemcpyAsync(dtiles + tiles[0].size(), tiles[1].data(), tiles[1].size() * sizeof(int4),
-                       hipMemcpyHostToDevice, st));
+  const size_t n0 = tiles[0].size(), n1 = tiles[1].size(), n2 = tiles[2].size();
+  tiles[0].insert(tiles[0].end(), tiles[1].begin(), tiles[1].end());
+  tiles[0].insert(tiles[0].end(), tiles[2].begin(), tiles[2].end());
+  HIPCK(hipMemcpyAsync(dtiles, tiles[0].data(), ntile * sizeof(int4), hipMemcpyHostToDevice, st));
   {
     PhaseScope ps(ctx, CDCLQ_PHASE_GRAM);
-    HIPCK(gram_mfma(st, djobs, dtiles, (int)tiles[0].size(), vec4));
-    HIPCK(gram_dma(st, djobs, dtiles + tiles[0].size(), (int)tiles[1].size(), prog));
+    HIPCK(gram_mfma(st, djobs, dtiles, (int)n0, vec4));
+    HIPCK(gram_dma(st, djobs, dtiles + n0, (int)n1, prog));
+    HIPCK(gram_parts(st, djobs, dtiles + n0 + n1, (int)n2));
   }
   HIPCK(hipStreamSynchronize(st));
   return CDCLQ_OK;

@@ -216,10 +216,18 @@ namespace cdclq {
 namespace {
 
 // xf = x * sqrt(w_t) per token (f32, as `xf * state["w"].sqrt().unsqueeze(1)`)
-__global__ __launch_bounds__(256) void k_token_scale(long t, int n, const float* __restrict__ x,
+// 2^lg threads to a row, V columns each (V = 4: 16-byte aligned rows).
+template <int V>
+__global__ __launch_bounds__(256) void k_token_scale(long t, int n, int lg, const float* __restrict__ x,
                                                      const float* __restrict__ w, float* __restrict__ out) {
-  for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < t * n; i += (long)gridDim.x * 256)
-    out[i] = x[i] * sqrtf(w[i / n]);
+  typedef float vec __attribute__((ext_vector_type(V)));
+  const int c0 = threadIdx.x & ((1 << lg) - 1), per = 256 >> lg;
+  for (long r = (long)blockIdx.x * per + (threadIdx.x >> lg); r < t; r += (long)gridDim.x * per) {
+    const float s = sqrtf(w[r]);
+    const vec* src = reinterpret_cast<const vec*>(x + r * n);
+    vec* dst = reinterpret_cast<vec*>(out + r * n);
+    for (int c = c0; c < n / V; c += 1 << lg) dst[c] = src[c] * s;
+  }
 }
 
 // h = (f32)(acc / count): the 1/N normalisation, rounded once from f64
@@ -233,9 +241,16 @@ __global__ __launch_bounds__(256) void k_normalize(long count, const double* __r
 
 hipError_t token_scale(hipStream_t st, long t, int n, const float* x, const float* w, float* out) {
   if (t * n <= 0) return hipSuccess;
-  // grid-stride: at most 2^20 workgroups, far below 2^32 work-items for any t x n
-  hipLaunchKernelGGL(k_token_scale, dim3((unsigned)std::min<long>((t * n + 255) / 256, 1L << 20)), dim3(256), 0, st,
-                     t, n, x, w, out);
+  const bool v4 = n % 4 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)out % 16 == 0;
+  const int nv = v4 ? n / 4 : n;
+  int lg = 8;
+  while (lg > 0 && (1 << (lg - 1)) >= nv) --lg;
+  // at most 2^20 workgroups, far below 2^32 work-items
+  const dim3 grid((unsigned)std::min<long>((t + (256 >> lg) - 1) / (256 >> lg), 1L << 20));
+  if (v4)
+    hipLaunchKernelGGL(k_token_scale<4>, grid, dim3(256), 0, st, t, n, lg, x, w, out);
+  else
+    hipLaunchKernelGGL(k_token_scale<1>, grid, dim3(256), 0, st, t, n, lg, x, w, out);
   return hipGetLastError();
 }
 

@@ -339,15 +339,126 @@ __global__ __launch_bounds__(512, 1) void k_gram_dma(const GramJob* __restrict__
   }
 }
 
-// flag |= (h not bitwise symmetric)
+// The tiles left over after whole rounds of 128 x 128 tiles (gram_dma_order), 16 workgroups of four
+// wavefronts to a tile: a workgroup owns 32 x 32 of it, a wavefront 16 x 16, and
+// v_mfma_f32_16x16x4_f32 adds four tokens a step, in ascending order with one rounding each. A
+// dependent chain of them keeps the matrix core busy with one wavefront per SIMD, so a tile's 16
+// workgroups take its work at the rate of 16 CUs where a 512-thread workgroup has one. Stages of 64 tokens
+// (X [64][32], then Y [64][32]) lie in a ring of four; two workgroups fit a CU. Arithmetic, order and folds
+// are those above. 4096 x 4096, 4096 tokens (528 tiles, 16 of them here): 849 -> 687 + 29 us.
+// Workgroup w runs on XCD w % 8: a tile's workgroups share its stripes in one L2.
+constexpr int SUB = 32;                    // side of a part
+constexpr int SPARTS = (TI / SUB) * (DTJ / SUB);
+constexpr int SRING = 4;
+constexpr int SSTAGE = DKT * 2 * SUB;      // floats per stage
+constexpr int SPW = SSTAGE / 256 / 4;      // 1 KB loads per wave and stage
+typedef float v4acc __attribute__((ext_vector_type(4)));
+
+__global__ __launch_bounds__(256) void k_gram_parts(const GramJob* __restrict__ jobs, const int4* __restrict__ tiles,
+                                                    int ntiles) {
+  __shared__ __attribute__((aligned(16))) float R[SRING * SSTAGE];
+  const int slot = blockIdx.x >> 3;
+  const int tile = (slot / SPARTS) * 8 + (blockIdx.x & 7), part = slot % SPARTS;
+  if (tile >= ntiles) return;
+  const int4 tl = tiles[tile];
+  const GramJob jb = jobs[tl.x];
+  const int n = jb.n, T = jb.t;
+  __attribute__((address_space(1))) double* H = (__attribute__((address_space(1))) double*)jb.h;
+  const int i0 = tl.y * TI + SUB * (part / (DTJ / SUB)), j0 = tl.z * DTJ + SUB * (part % (DTJ / SUB));
+  const bool mirror = (tl.w & 1) != 0;
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wr = wv >> 1, wc = wv & 1;
+  const int row = i0 + 16 * wr + 4 * (lane >> 4), col = j0 + 16 * wc + (lane & 15);
+  double h[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) h[r] = H[(long)(row + r) * n + col];
+  const float* src[SPW];
+#pragma unroll
+  for (int q = 0; q < SPW; ++q) {  // instruction i: tokens 8 (i & 7) + (lane >> 3), columns 4 (lane & 7)
+    const int ins = wv + 4 * q;
+    src[q] = (ins < 8 ? jb.x + i0 : jb.y + j0) + (long)(8 * (ins & 7) + (lane >> 3)) * n + 4 * (lane & 7);
+  }
+  const uint32_t base = lds_offset(R);
+  const int nstage = T / DKT;
+  auto issue = [&](int s) {
+    const long t0n = (long)s * DKT * n;
+#pragma unroll
+    for (int q = 0; q < SPW; ++q)
+      dma16_untracked(src[q] + t0n, base + 4u * (uint32_t)(SSTAGE * (s % SRING) + 256 * (wv + 4 * q)));
+  };
+  for (int s = 0; s < min(SRING - 1, nstage); ++s) issue(s);
+  v4acc acc = {};
+  float tmp[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  for (int s = 0; s < nstage; ++s) {
+    // this wave's part of stage s has landed; the barrier publishes every wave's part and retires all
+    // reads of stage s - 1, whose place in the ring stage s + 3 then takes
+    if (s + 2 < nstage) wait_vmcnt<2 * SPW>();
+    else if (s + 1 < nstage) wait_vmcnt<SPW>();
+    else wait_vmcnt<0>();
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (s + SRING - 1 < nstage) issue(s + SRING - 1);
+    const float* xs = R + SSTAGE * (s % SRING) + (lane >> 4) * SUB + 16 * wr + (lane & 15);
+    const float* ys = R + SSTAGE * (s % SRING) + DKT * SUB + (lane >> 4) * SUB + 16 * wc + (lane & 15);
+    float a[DKT / 4], b[DKT / 4];
+#pragma unroll
+    for (int p = 0; p < DKT / 4; ++p) {
+      a[p] = xs[4 * p * SUB];
+      b[p] = ys[4 * p * SUB];
+    }
+#pragma unroll
+    for (int p = 0; p < DKT / 4; ++p) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[p], b[p], acc, 0, 0, 0);
+    // issue order: reads (two steps of an operand each) run four steps ahead of the matrix core
+    __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+#pragma unroll
+    for (int p = 0; p < DKT / 4 - 4; ++p) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
+    const int tn = (s + 1) * DKT;
+    if ((tn % CDCLQ_KC) == 0 || tn >= T) {  // panel end
+#pragma unroll
+      for (int r = 0; r < 4; ++r) tmp[r] = __builtin_fmaf(1.0f, acc[r], tmp[r]);
+      acc = v4acc{};
+      if ((tn % 2048) == 0 || tn >= T) {  // chunk end
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          h[r] += (double)tmp[r];
+          tmp[r] = 0.0f;
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    H[(long)(row + r) * n + col] = h[r];
+    if (mirror) H[(long)col * n + row + r] = h[r];
+  }
+}
+
+// flag |= (h not bitwise symmetric): workgroup (x, y) compares block (y, x) of 64 x 64 with the
+// transpose of block (x, y), turned in LDS so that both are read along their rows. 4096 x 4096:
+// 23 us (an element and its counterpart per thread: 74 us).
 __global__ __launch_bounds__(256) void k_sym_check(int n, const double* __restrict__ h, int* flag) {
-  const long idx = (long)blockIdx.x * 256 + threadIdx.x;
-  if (idx >= (long)n * n) return;
-  const int i = (int)(idx / n), j = (int)(idx % n);
-  if (j <= i) return;
-  const unsigned long long a = __double_as_longlong(h[idx]);
-  const unsigned long long b = __double_as_longlong(h[(long)j * n + i]);
-  if (a != b) atomicOr(flag, 1);
+  __shared__ unsigned long long t[64][65];
+  if (blockIdx.x < blockIdx.y) return;
+  const int i0 = 64 * blockIdx.y, j0 = 64 * blockIdx.x;
+  const int c = threadIdx.x & 63, r0 = threadIdx.x >> 6;
+  const unsigned long long* hb = reinterpret_cast<const unsigned long long*>(h);
+  unsigned long long u[16], v[16];
+#pragma unroll
+  for (int q = 0; q < 16; ++q) {  // clamped: rows and columns past n repeat the last, on both sides
+    const int r = r0 + 4 * q;
+    v[q] = hb[(long)min(j0 + r, n - 1) * n + min(i0 + c, n - 1)];
+    u[q] = hb[(long)min(i0 + r, n - 1) * n + min(j0 + c, n - 1)];
+  }
+#pragma unroll
+  for (int q = 0; q < 16; ++q) t[r0 + 4 * q][c] = v[q];
+  __syncthreads();
+  bool differ = false;
+#pragma unroll
+  for (int q = 0; q < 16; ++q) differ |= u[q] != t[c][r0 + 4 * q];
+  if (__builtin_amdgcn_ballot_w64(differ) && (threadIdx.x & 63) == 0) atomicOr(flag, 1);
 }
 
 // A fill kernel rather than hipMemsetAsync, so the clear stays an ordinary kernel node when a
@@ -392,6 +503,12 @@ hipError_t gram_dma(hipStream_t st, const GramJob* jobs, const int4* tiles, int 
   return hipGetLastError();
 }
 
+hipError_t gram_parts(hipStream_t st, const GramJob* jobs, const int4* tiles, int ntiles) {
+  if (ntiles <= 0) return hipSuccess;
+  hipLaunchKernelGGL(k_gram_parts, dim3((ntiles + 7) / 8 * 8 * SPARTS), dim3(256), 0, st, jobs, tiles, ntiles);
+  return hipGetLastError();
+}
+
 // Morton index of tile (I, J), the column bit lowest: 32 consecutive indices are a 4 x 8 block
 static uint64_t tile_morton(int I, int J) {
   uint64_t k = 0;
@@ -399,7 +516,7 @@ static uint64_t tile_morton(int I, int J) {
   return k;
 }
 
-void gram_dma_order(std::vector<int4>& tl) {
+void gram_dma_order(int cus, std::vector<int4>& tl, std::vector<int4>& rest) {
   // each job's tiles in Morton order, jobs one after another
   for (size_t i = 0; i < tl.size();) {
     size_t j = i;
@@ -407,6 +524,14 @@ void gram_dma_order(std::vector<int4>& tl) {
     std::stable_sort(tl.begin() + i, tl.begin() + j,
                      [](const int4& a, const int4& b) { return tile_morton(a.y, a.z) < tile_morton(b.y, b.z); });
     i = j;
+  }
+  // A last round of at most half the CUs goes to k_gram_parts: its time there grows with the tiles, against
+  // a whole round here whatever their number (4096 tokens: 16 tiles 29 us, 36 50 us, 66 100 us; a round of 256
+  // 340 us, of 16 160 us).
+  const size_t last = tl.size() % (size_t)cus;
+  if (2 * last <= (size_t)cus) {
+    rest.assign(tl.end() - last, tl.end());
+    tl.resize(tl.size() - last);
   }
   // gangs of 32 consecutive tiles (one may span two jobs), so the launch takes no more rounds of
   // 256 workgroups than the tiles need; the gang fields stay 0 (no pacing) past 2^19 gangs
@@ -458,8 +583,8 @@ hipError_t zero_words(hipStream_t st, int* p, int count) {
 }
 
 hipError_t sym_check(hipStream_t st, int n, const double* h, int* flag) {
-  const long nn = (long)n * n;
-  hipLaunchKernelGGL(k_sym_check, dim3((unsigned)((nn + 255) / 256)), dim3(256), 0, st, n, h, flag);
+  const unsigned nb = (unsigned)((n + 63) / 64);
+  hipLaunchKernelGGL(k_sym_check, dim3(nb, nb), dim3(256), 0, st, n, h, flag);
   return hipGetLastError();
 }
 

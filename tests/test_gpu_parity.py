@@ -181,6 +181,20 @@ def test_gram_batch_matches_single_calls(ctx):
         assert np.array_equal(d.download().view(np.uint64), ho.view(np.uint64)), (t, n)
 
 
+@pytest.mark.parametrize("t,n,sym", [(320, 2944, True), (320, 2176, False), (2112, 1536, False), (4160, 640, True)])
+def test_gram_whole_rounds_and_rest(ctx, t, n, sym):
+    """Tiles of 128 x 128 beyond whole rounds of the device: 256 + 20, 256 + 33, 144 (a round of its own) and
+    15 (none) of them on 256 CUs; token counts that end inside a panel and after a chunk."""
+    rng = np.random.default_rng(t + n)
+    x = (rng.standard_normal((t, n)) * rng.uniform(0.1, 10, n)).astype(np.float32)
+    y = x if sym else (x + 0.05 * rng.standard_normal((t, n))).astype(np.float32)
+    h0 = np.zeros((n, n)) if sym else rng.standard_normal((n, n))
+    hg = h0.copy()
+    cdclq.gram_accumulate(x, y, t, n, hg, ctx)
+    ho = O.gram_accumulate(x, None if sym else y, h0.copy())
+    assert np.array_equal(hg.view(np.uint64), ho.view(np.uint64))
+
+
 def test_gram_batch_gangs_across_jobs(ctx):
     """Direct-to-LDS jobs of different widths and token counts in one launch: 132 tiles in gangs of
     32, two gangs spanning two jobs (members with different token counts pace each other until the
