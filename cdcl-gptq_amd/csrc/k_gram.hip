@@ -345,7 +345,8 @@ __global__ __launch_bounds__(512, 1) void k_gram_dma(const GramJob* __restrict__
 // dependent chain of them keeps the matrix core busy with one wavefront per SIMD, so a tile's 16
 // workgroups take its work at the rate of 16 CUs where a 512-thread workgroup has one. Stages of 64 tokens
 // (X [64][32], then Y [64][32]) lie in a ring of four; two workgroups fit a CU. Arithmetic, order and folds
-// are those above. 4096 x 4096, 4096 tokens (528 tiles, 16 of them here): 849 -> 687 + 29 us.
+// are those above. 4096 x 4096, 4096 tokens (528 tiles, 16 of them here): 849 -> 687 + 29 us
+// (with pacing; 631 + 30 without).
 // Workgroup w runs on XCD w % 8: a tile's workgroups share its stripes in one L2.
 constexpr int SUB = 32;                    // side of a part
 constexpr int SPARTS = (TI / SUB) * (DTJ / SUB);
@@ -527,7 +528,7 @@ void gram_dma_order(int cus, std::vector<int4>& tl, std::vector<int4>& rest) {
   }
   // A last round of at most half the CUs goes to k_gram_parts: its time there grows with the tiles, against
   // a whole round here whatever their number (4096 tokens: 16 tiles 29 us, 36 50 us, 66 100 us; a round of 256
-  // 340 us, of 16 160 us).
+  // 280 us, of 16 160 us).
   const size_t last = tl.size() % (size_t)cus;
   if (2 * last <= (size_t)cus) {
     rest.assign(tl.end() - last, tl.end());
