@@ -162,17 +162,13 @@ int pack_device(cdclq_ctx* ctx, size_t d_out, size_t n, size_t g, const uint8_t*
   const bool runs = (g % 8 == 0) || (n <= g);
   {
     PhaseScope ps(ctx, CDCLQ_PHASE_PACK);
-    if (runs) {
+    if (runs)
       HIPCK(pack_runs(ctx->st, (long)d_out, (int)n, (int)L.rb, codes, D.rdesc, qweight, spill, epoch));
-      // a code wider than its group's width spills into the next run: then the general kernel,
-      // which follows the reference's unmasked OR, redoes the layer (a no-op launch otherwise)
-      HIPCK(pack_rows(ctx->st, (long)d_out, (int)n, (int)L.rb, codes, D.coff, D.wfirst, qweight, spill, epoch));
-    } else {
-      HIPCK(pack_rows(ctx->st, (long)d_out, (int)n, (int)L.rb, codes, D.coff, D.wfirst, qweight, nullptr, 0));
-    }
-    HIPCK(pack_meta(ctx->st, (long)(d_out * ng), scales, zeros, s16, qz));
+    // a code wider than its group's width spills into the next run: then the general path, which
+    // follows the reference's unmasked OR, redoes the layer
+    HIPCK(pack_rest(ctx->st, (long)d_out, (int)n, (int)L.rb, codes, D.coff, D.wfirst, qweight, runs ? spill : nullptr,
+                    epoch, (long)(d_out * ng), scales, zeros, s16, qz, perm, reinterpret_cast<uint32_t*>(p32)));
   }
-  HIPCK(hipMemcpyAsync(p32, perm, n * 4, hipMemcpyDeviceToDevice, ctx->st));  // `p as i32`: same bits
   HIPCK(hipStreamSynchronize(ctx->st));
   return CDCLQ_OK;
 }

@@ -84,19 +84,11 @@ __device__ __forceinline__ uint8_t f32_as_u8(float z) {
   return (uint8_t)z;
 }
 
-// One thread per 4-byte word of a row: word w holds row bits [32 w, 32 w + 32). `coff[j]` is
-// off_j (j <= n, coff[n] = total bits); `wfirst[w]` the first code whose 8-bit window
-// [off_j, off_j + 8) reaches bit 32 w.
-// With `only_if` set the kernel does nothing unless *only_if == epoch (the fast path's spill flag
-// of this call), so the fallback can be enqueued without a host round trip.
-__global__ __launch_bounds__(256) void k_pack_rows(long d_out, int n, int rb, int wpr, const uint8_t* __restrict__ codes,
-                                                   const uint32_t* __restrict__ coff,
-                                                   const int* __restrict__ wfirst, uint8_t* __restrict__ qw,
-                                                   const uint32_t* __restrict__ only_if, uint32_t epoch) {
-  if (only_if && *only_if != epoch) return;
-  for (long t = (long)blockIdx.x * 256 + threadIdx.x; t < d_out * wpr; t += (long)gridDim.x * 256) {
-  const long r = t / wpr;
-  const int w = (int)(t - r * wpr);
+// Word w of row r: row bits [32 w, 32 w + 32). `coff[j]` is off_j (j <= n, coff[n] = total bits);
+// `wfirst[w]` the first code whose 8-bit window [off_j, off_j + 8) reaches bit 32 w.
+__device__ __forceinline__ void pack_word(long r, int w, int n, int rb, const uint8_t* __restrict__ codes,
+                                          const uint32_t* __restrict__ coff, const int* __restrict__ wfirst,
+                                          uint8_t* __restrict__ qw) {
   const uint8_t* cr = codes + r * n;
   const int bit0 = 32 * w;
   uint64_t v = 0;
@@ -115,17 +107,31 @@ __global__ __launch_bounds__(256) void k_pack_rows(long d_out, int n, int rb, in
     for (int k = 0; k < 4; ++k)
       if (4 * w + k < rb) dst[k] = (uint8_t)(v >> (8 * k));
   }
-  }
 }
 
-// .scales (f16 bits) and .qzeros (u8) of io::packed_tensors (src/io.rs:250-256).
-__global__ __launch_bounds__(256) void k_pack_meta(long count, const float* __restrict__ scales,
-                                                   const float* __restrict__ zeros, uint16_t* __restrict__ s16,
-                                                   uint8_t* __restrict__ z8) {
-  const long i = (long)blockIdx.x * 256 + threadIdx.x;
-  if (i >= count) return;
-  s16[i] = f32_to_f16_bits(scales[i]);
-  z8[i] = f32_as_u8(zeros[i]);
+// What follows the fast path of the codes, in one launch: the companion tensors, .scales (f16 bits)
+// and .qzeros (u8) of io::packed_tensors (src/io.rs:250-256), the permutation (`p as i32`: same
+// bits), and the code rows by words. The rows are packed only if *only_if == epoch, the fast path's
+// spill flag of this call (no host round trip), or if only_if is null. Launches and a copy, not
+// bytes, bound this part of a call: @@T1@@
+__global__ __launch_bounds__(256) void k_pack_rest(long d_out, int n, int rb, int wpr, const uint8_t* __restrict__ codes,
+                                                   const uint32_t* __restrict__ coff,
+                                                   const int* __restrict__ wfirst, uint8_t* __restrict__ qw,
+                                                   const uint32_t* __restrict__ only_if, uint32_t epoch, long nmeta,
+                                                   const float* __restrict__ scales, const float* __restrict__ zeros,
+                                                   uint16_t* __restrict__ s16, uint8_t* __restrict__ z8,
+                                                   const uint32_t* perm, uint32_t* p32) {
+  const long t0 = (long)blockIdx.x * 256 + threadIdx.x, step = (long)gridDim.x * 256;
+  for (long i = t0; i < nmeta; i += step) {
+    s16[i] = f32_to_f16_bits(scales[i]);
+    z8[i] = f32_as_u8(zeros[i]);
+  }
+  for (long i = t0; i < n; i += step) p32[i] = perm[i];
+  if (only_if && *only_if != epoch) return;
+  for (long t = t0; t < d_out * wpr; t += step) {
+    const long r = t / wpr;
+    pack_word(r, (int)(t - r * wpr), n, rb, codes, coff, wfirst, qw);
+  }
 }
 
 // Inverse column map with the reference's scatter semantics (`row[perm[j]] = ...`, later j wins,
@@ -149,18 +155,14 @@ __global__ __launch_bounds__(256) void k_invert_perm(int n, const uint32_t* __re
   atomicMax(&last[c], j);
 }
 
-// Per output column c, in the form the dequantization consumes: cdesc[c] = byte offset in a staged
-// row of the aligned 64-bit word holding the first bit of column last[c]'s code (bits 0-19), the
-// bit position in that word (bits 20-25) and the code width (bits 26-29); unpacked rows hold one
-// byte per code, so there it is the byte offset last[c] with width 8. cgrp[c] = byte offset of the
-// column's (scale, zero) pair in a staged row's pairs. Bit 31 of cdesc marks a column that no j
-// writes.
-__global__ __launch_bounds__(256) void k_col_desc(int n, int g, int packed, const int* __restrict__ last,
-                                                  const uint32_t* __restrict__ coff, const uint8_t* __restrict__ cwid,
-                                                  uint32_t* __restrict__ cdesc, int* __restrict__ cgrp) {
-  const int c = blockIdx.x * 256 + threadIdx.x;
-  if (c >= n) return;
-  const int j = last[c];
+// Column c's entry, in the form the dequantization consumes, for j = last[c]: cdesc[c] = byte offset
+// in a staged row of the aligned 64-bit word holding the first bit of code j (bits 0-19), the bit
+// position in that word (bits 20-25) and the code width (bits 26-29); unpacked rows hold one byte
+// per code, so there it is the byte offset j with width 8. cgrp[c] = byte offset of the column's
+// (scale, zero) pair in a staged row's pairs. Bit 31 of cdesc marks a column that no j writes.
+__device__ __forceinline__ void column_entry(int c, int j, int g, int packed, const uint32_t* __restrict__ coff,
+                                             const uint8_t* __restrict__ cwid, uint32_t* __restrict__ cdesc,
+                                             int* __restrict__ cgrp) {
   if (j < 0) {
     cdesc[c] = 0x80000000u;
     cgrp[c] = 0;
@@ -173,6 +175,45 @@ __global__ __launch_bounds__(256) void k_col_desc(int n, int g, int packed, cons
     cdesc[c] = (uint32_t)j | (8u << 26);
   }
   cgrp[c] = (j / g) * 8;
+}
+
+__global__ __launch_bounds__(256) void k_col_desc(int n, int g, int packed, const int* __restrict__ last,
+                                                  const uint32_t* __restrict__ coff, const uint8_t* __restrict__ cwid,
+                                                  uint32_t* __restrict__ cdesc, int* __restrict__ cgrp) {
+  const int c = blockIdx.x * 256 + threadIdx.x;
+  if (c < n) column_entry(c, last[c], g, packed, coff, cwid, cdesc, cgrp);
+}
+
+// The whole map in one launch: a workgroup of 1024 threads owns 256 columns, reads every entry of
+// perm (from L2, eight per thread in flight) and keeps its columns' last writer in LDS. The three
+// launches it replaces (fill, inversion, entries) are bound by their latency: @@T2@@
+__global__ __launch_bounds__(1024) void k_col_map(int n, int g, int packed, const uint32_t* __restrict__ perm,
+                                                  const uint32_t* __restrict__ coff, const uint8_t* __restrict__ cwid,
+                                                  uint32_t* __restrict__ cdesc, int* __restrict__ cgrp,
+                                                  uint32_t* __restrict__ bad, uint32_t epoch) {
+  __shared__ int last[256];
+  const int tid = threadIdx.x;
+  const uint32_t c0 = blockIdx.x * 256u;
+  if (tid < 256) last[tid] = -1;
+  __syncthreads();
+  for (int j0 = tid; j0 < n; j0 += 8192) {
+    uint32_t c[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) c[q] = perm[min(j0 + 1024 * q, n - 1)];  // clamped: loads never branch
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const int j = j0 + 1024 * q;
+      if (j >= n) break;
+      if (c[q] >= (uint32_t)n) {
+        if (blockIdx.x == 0) atomicExch(bad, epoch);
+      } else if (c[q] - c0 < 256u) {  // wraps to a large value below c0
+        atomicMax(&last[c[q] - c0], j);
+      }
+    }
+  }
+  __syncthreads();
+  const int c = (int)c0 + tid;
+  if (tid < 256 && c < n) column_entry(c, last[tid], g, packed, coff, cwid, cdesc, cgrp);
 }
 
 typedef float f32x2 __attribute__((ext_vector_type(2)));
@@ -343,7 +384,7 @@ __global__ __launch_bounds__(256) void k_dequant_rows(long d_out, int rpb, int n
 // and fills exactly b bytes (the row's last, shorter run ends in the zero-filled partial byte).
 // One thread per run. A code wider than its group's width would spill into the next run's bits
 // (the reference ORs whole u8 codes); such a row is flagged in *spill and the caller re-packs the
-// layer with k_pack_rows, which follows the reference for any input.
+// layer with pack_word, which follows the reference for any input.
 // rdesc[k] = (byte offset of run k) << 4 | its width.
 __global__ __launch_bounds__(256) void k_pack_runs(long d_out, int n, int rb, int runs, const uint8_t* __restrict__ codes,
                                                    const uint32_t* __restrict__ rdesc, uint8_t* __restrict__ qw,
@@ -386,27 +427,27 @@ __global__ __launch_bounds__(256) void k_pack_runs(long d_out, int n, int rb, in
 
 }  // namespace
 
-hipError_t pack_rows(hipStream_t st, long d_out, int n, int rb, const uint8_t* codes, const uint32_t* coff,
-                     const int* wfirst, uint8_t* qw, const uint32_t* only_if, uint32_t epoch) {
+hipError_t pack_rest(hipStream_t st, long d_out, int n, int rb, const uint8_t* codes, const uint32_t* coff,
+                     const int* wfirst, uint8_t* qw, const uint32_t* only_if, uint32_t epoch, long nmeta,
+                     const float* scales, const float* zeros, uint16_t* s16, uint8_t* z8, const uint32_t* perm,
+                     uint32_t* p32) {
   const int wpr = (rb + 3) / 4;
-  const long total = d_out * wpr;
-  if (total <= 0) return hipSuccess;
-  const long blocks = std::min<long>((total + 255) / 256, 2048);
-  hipLaunchKernelGGL(k_pack_rows, dim3((unsigned)blocks), dim3(256), 0, st, d_out, n, rb, wpr, codes, coff, wfirst, qw,
-                     only_if, epoch);
-  return hipGetLastError();
-}
-
-hipError_t pack_meta(hipStream_t st, long count, const float* scales, const float* zeros, uint16_t* s16, uint8_t* z8) {
-  if (count <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_pack_meta, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, st, count, scales, zeros, s16,
-                     z8);
+  const long most = std::max(std::max(d_out * wpr, nmeta), (long)n);
+  const long blocks = std::min<long>((most + 255) / 256, 2048);
+  hipLaunchKernelGGL(k_pack_rest, dim3((unsigned)blocks), dim3(256), 0, st, d_out, n, rb, wpr, codes, coff, wfirst, qw,
+                     only_if, epoch, nmeta, scales, zeros, s16, z8, perm, p32);
   return hipGetLastError();
 }
 
 hipError_t column_map(hipStream_t st, int n, int g, bool packed, const uint32_t* perm, const uint32_t* coff,
                       const uint8_t* cwid, int* last, uint32_t* cdesc, int* cgrp, uint32_t* bad, uint32_t epoch) {
   const dim3 grid((unsigned)((n + 255) / 256));
+  // k_col_map reads perm once per 256 columns: @@T3@@
+  if (n <= 32768) {
+    hipLaunchKernelGGL(k_col_map, grid, dim3(1024), 0, st, n, g, packed ? 1 : 0, perm, coff, cwid, cdesc, cgrp, bad,
+                       epoch);
+    return hipGetLastError();
+  }
   hipLaunchKernelGGL(k_fill_i32, grid, dim3(256), 0, st, n, -1, last);
   hipLaunchKernelGGL(k_invert_perm, grid, dim3(256), 0, st, n, perm, last, bad, epoch);
   hipLaunchKernelGGL(k_col_desc, grid, dim3(256), 0, st, n, g, packed ? 1 : 0, last, coff, cwid, cdesc, cgrp);

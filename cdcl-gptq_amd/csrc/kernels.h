@@ -216,15 +216,17 @@ hipError_t pass_accum(hipStream_t st, int rows, int rc, int nchunks, int nref, c
                       const uint8_t* active, double* ld, uint64_t* upd);
 // ---- k_pack.hip: packed container cdclq-v1 (bit streams LSB first, per-group widths)
 // qw (d_out x rb) from codes (d_out x n); coff[j] = bit offset of code j (coff[n] = total bits),
-// wfirst[w] = first code whose 8-bit window reaches bit 32 w of a row. With only_if non-null the
-// launch does nothing unless *only_if == epoch.
-hipError_t pack_rows(hipStream_t st, long d_out, int n, int rb, const uint8_t* codes, const uint32_t* coff,
-                     const int* wfirst, uint8_t* qw, const uint32_t* only_if, uint32_t epoch);
+// wfirst[w] = first code whose 8-bit window reaches bit 32 w of a row. With only_if non-null the rows
+// are left alone unless *only_if == epoch. The same launch writes the companion tensors (nmeta scales
+// as f16 and zeros as u8) and the n entries of the permutation.
+hipError_t pack_rest(hipStream_t st, long d_out, int n, int rb, const uint8_t* codes, const uint32_t* coff,
+                     const int* wfirst, uint8_t* qw, const uint32_t* only_if, uint32_t epoch, long nmeta,
+                     const float* scales, const float* zeros, uint16_t* s16, uint8_t* z8, const uint32_t* perm,
+                     uint32_t* p32);
 // fast path when every run of 8 columns lies in one group (rdesc[k] = byte offset of run k << 4 |
-// width); *spill is set to epoch if a code exceeds its width (then pack_rows redoes the layer)
+// width); *spill is set to epoch if a code exceeds its width (then pack_rest redoes the layer)
 hipError_t pack_runs(hipStream_t st, long d_out, int n, int rb, const uint8_t* codes, const uint32_t* rdesc,
                      uint8_t* qw, uint32_t* spill, uint32_t epoch);
-hipError_t pack_meta(hipStream_t st, long count, const float* scales, const float* zeros, uint16_t* s16, uint8_t* z8);
 // output column map: last[c] = max j with perm[j] == c (-1: none), cdesc[c] = bit offset << 4 |
 // width (packed) or last[c] (unpacked), cgrp[c] = last[c] / g; *bad is set to epoch if some
 // perm[j] >= n.

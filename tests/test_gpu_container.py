@@ -183,6 +183,25 @@ def test_repeated_perm_entries_keep_the_scatter_result(ctx):
     _same_bits(got, O.dequantize_packed(qw, s16, qz, p32, ql.gbits, 128, "F32"), "dup perm")
 
 
+@pytest.mark.parametrize("n", [255, 256, 257, 8191, 8193, 32768, 32769])
+def test_column_map_edges(ctx, n):
+    """Ends of the map's 256-column workgroups and 8192-entry rounds, and both sides of the width up to
+    which it is one launch; with entries repeated across rounds, and one past the end refused."""
+    ql = _layer(n, 128, 3, n)
+    ql.perm[n - 1] = ql.perm[0]
+    ql.perm[n // 2] = ql.perm[n // 3]
+    qw, s16, qz, p32 = _oracle_pack(ql)
+    got = cdclq.dequantize_packed(ctx, qw, s16, qz, p32, ql.gbits, 128, "F32")
+    _same_bits(got, O.dequantize_packed(qw, s16, qz, p32, ql.gbits, 128, "F32"), f"n={n}")
+    ref32 = O.QLayer(3, n, 128, ql.perm, ql.gbits, ql.codes, ql.scales, ql.zeros, {}).dequantize()
+    _same_bits(cdclq.dequantize_layer(ctx, ql, "F32"), ref32, f"unpacked n={n}")
+    for a, b in zip(cdclq.pack_layer(ctx, ql), (qw, s16, qz, p32)):
+        _same_bits(a, b, f"pack n={n}")
+    p32[n - 1] = n
+    with pytest.raises(cdclq.CdclqError):
+        cdclq.dequantize_packed(ctx, qw, s16, qz, p32, ql.gbits, 128, "F32")
+
+
 def test_device_entry_points_match_host(ctx):
     ql = _layer(4096, 128, 40, 9, gb=[4] * 32)
     d_out, n, g, ng = ql.d_out, ql.d_in, ql.group, ql.ngroups()
