@@ -7,6 +7,7 @@
 //             whole u8 code can reach 8 bits past its offset, src/quant.rs:120).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstring>
 #include <string>
 #include <vector>
@@ -85,17 +86,19 @@ struct LayoutDev {
 };
 
 // Uploads the tables into ctx->pk_tab[0] as one block: coff (n+1 u32) | wfirst (wpr i32) |
-// rdesc (runs u32) | cwid (n u8). The block stays valid for later calls with the same layout (every
-// call ends with a stream synchronisation, so no kernel still reads it when it is replaced).
-int upload_layout(cdclq_ctx* ctx, const Layout& L, size_t g, LayoutDev* D) {
-  const size_t n = L.cwid.size();
-  const size_t a = (L.coff.size() * 4 + 255) & ~(size_t)255;
-  const size_t b = (L.wfirst.size() * 4 + 255) & ~(size_t)255;
-  const size_t c = (L.rdesc.size() * 4 + 255) & ~(size_t)255;
-  char* base;
+// rdesc (runs u32) | cwid (n u8). The block stays valid for later calls with the same n, g and group
+// widths, which then build nothing either (every call ends with a stream synchronisation, so no
+// kernel still reads it when it is replaced).
+int upload_layout(cdclq_ctx* ctx, size_t n, size_t g, const uint8_t* gbits, LayoutDev* D) {
+  const size_t used = (n + g - 1) / g, wpr = (row_bytes_of(n, g, gbits) + 3) / 4;
+  const size_t a = ((n + 1) * 4 + 255) & ~(size_t)255;
+  const size_t b = (wpr * 4 + 255) & ~(size_t)255;
+  const size_t c = ((n + 7) / 8 * 4 + 255) & ~(size_t)255;
   const bool hit = ctx->pk_layout_valid && ctx->pk_layout_n == n && ctx->pk_layout_g == g &&
-                   ctx->pk_layout_wid == L.cwid && ctx->pk_tab[0].p != nullptr;
+                   std::equal(ctx->pk_layout_wid.begin(), ctx->pk_layout_wid.end(), gbits, gbits + used) &&
+                   ctx->pk_tab[0].p != nullptr;
   if (!hit) {
+    const Layout L = build_layout(n, g, gbits);
     ctx->pk_layout_valid = false;
     std::vector<char> blob(a + b + c + n + 16, 0);
     std::memcpy(blob.data(), L.coff.data(), L.coff.size() * 4);
@@ -107,9 +110,9 @@ int upload_layout(cdclq_ctx* ctx, const Layout& L, size_t g, LayoutDev* D) {
     ctx->pk_layout_valid = true;
     ctx->pk_layout_n = n;
     ctx->pk_layout_g = g;
-    ctx->pk_layout_wid = L.cwid;
+    ctx->pk_layout_wid.assign(gbits, gbits + used);
   }
-  base = P<char>(ctx->pk_tab[0]);
+  char* base = P<char>(ctx->pk_tab[0]);
   D->coff = reinterpret_cast<uint32_t*>(base);
   D->wfirst = reinterpret_cast<int*>(base + a);
   D->rdesc = reinterpret_cast<uint32_t*>(base + a + b);
@@ -148,13 +151,13 @@ int pack_device(cdclq_ctx* ctx, size_t d_out, size_t n, size_t g, const uint8_t*
   if (!why.empty()) return fail(ctx, CDCLQ_INVALID_ARG, why);
   if (!codes || !scales || !zeros || !perm || !qweight || !s16 || !qz || !p32)
     return fail(ctx, CDCLQ_INVALID_ARG, "null buffer argument");
-  const Layout L = build_layout(n, g, gbits);
-  if (qweight_bytes < d_out * L.rb)
+  const size_t rb = row_bytes_of(n, g, gbits);
+  if (qweight_bytes < d_out * rb)
     return fail(ctx, CDCLQ_INVALID_ARG, "qweight holds " + std::to_string(qweight_bytes) + " bytes, the layer needs " +
-                                            std::to_string(d_out * L.rb));
+                                            std::to_string(d_out * rb));
   HIPCK(hipSetDevice(ctx->device));
   LayoutDev D;
-  CK(upload_layout(ctx, L, g, &D));
+  CK(upload_layout(ctx, n, g, gbits, &D));
   CK(flags(ctx));
   uint32_t* spill = P<uint32_t>(ctx->pk_flag) + 1;
   const uint32_t epoch = next_epoch(ctx);
@@ -163,10 +166,10 @@ int pack_device(cdclq_ctx* ctx, size_t d_out, size_t n, size_t g, const uint8_t*
   {
     PhaseScope ps(ctx, CDCLQ_PHASE_PACK);
     if (runs)
-      HIPCK(pack_runs(ctx->st, (long)d_out, (int)n, (int)L.rb, codes, D.rdesc, qweight, spill, epoch));
+      HIPCK(pack_runs(ctx->st, (long)d_out, (int)n, (int)rb, codes, D.rdesc, qweight, spill, epoch));
     // a code wider than its group's width spills into the next run: then the general path, which
     // follows the reference's unmasked OR, redoes the layer
-    HIPCK(pack_rest(ctx->st, (long)d_out, (int)n, (int)L.rb, codes, D.coff, D.wfirst, qweight, runs ? spill : nullptr,
+    HIPCK(pack_rest(ctx->st, (long)d_out, (int)n, (int)rb, codes, D.coff, D.wfirst, qweight, runs ? spill : nullptr,
                     epoch, (long)(d_out * ng), scales, zeros, s16, qz, perm, reinterpret_cast<uint32_t*>(p32)));
   }
   HIPCK(hipStreamSynchronize(ctx->st));
@@ -193,10 +196,12 @@ int map_columns(cdclq_ctx* ctx, size_t n, size_t g, bool packed, const uint32_t*
 // Waits for the dequantization and reports a perm entry outside 0..n (the reference panics on its
 // out-of-bounds scatter; here the output is unspecified and the call fails).
 int finish_dequant(cdclq_ctx* ctx, size_t n) {
-  uint32_t bad = 0;
-  HIPCK(hipMemcpyAsync(&bad, ctx->pk_flag.p, 4, hipMemcpyDeviceToHost, ctx->st));
+  // through pinned memory: a copy to the stack stages it and waits for the stream a second time
+  CK(ensure_pinned(ctx, 16));
+  uint32_t* bad = static_cast<uint32_t*>(ctx->pin);
+  HIPCK(hipMemcpyAsync(bad, ctx->pk_flag.p, 4, hipMemcpyDeviceToHost, ctx->st));
   HIPCK(hipStreamSynchronize(ctx->st));
-  if (bad == ctx->pk_epoch)
+  if (*bad == ctx->pk_epoch)
     return fail(ctx, CDCLQ_INVALID_ARG, "perm has an entry outside 0..d_in (" + std::to_string(n) + ")");
   return CDCLQ_OK;
 }
@@ -209,19 +214,19 @@ int dequant_packed_device(cdclq_ctx* ctx, size_t d_out, size_t n, size_t g, cons
   const std::string why = check_layout(n, g, gbits, ng, true);
   if (!why.empty()) return fail(ctx, CDCLQ_INVALID_ARG, why);
   if (!qweight || !s16 || !qz || !p32 || !out) return fail(ctx, CDCLQ_INVALID_ARG, "null buffer argument");
-  const Layout L = build_layout(n, g, gbits);
-  if (qweight_bytes < d_out * L.rb)
+  const size_t rb = row_bytes_of(n, g, gbits);
+  if (qweight_bytes < d_out * rb)
     return fail(ctx, CDCLQ_INVALID_ARG, "qweight holds " + std::to_string(qweight_bytes) + " bytes, the layer needs " +
-                                            std::to_string(d_out * L.rb));
+                                            std::to_string(d_out * rb));
   HIPCK(hipSetDevice(ctx->device));
   LayoutDev D;
-  CK(upload_layout(ctx, L, g, &D));
+  CK(upload_layout(ctx, n, g, gbits, &D));
   uint32_t* cdesc;
   int* cgrp;
   CK(map_columns(ctx, n, g, true, reinterpret_cast<const uint32_t*>(p32), D.coff, D.cwid, &cdesc, &cgrp));
   {
     PhaseScope ps(ctx, CDCLQ_PHASE_DEQUANT);
-    HIPCK(dequant_rows(ctx->st, true, dtype, (long)d_out, (int)n, (int)ng, (int)L.rb, qweight, cdesc, cgrp, s16, qz,
+    HIPCK(dequant_rows(ctx->st, true, dtype, (long)d_out, (int)n, (int)ng, (int)rb, qweight, cdesc, cgrp, s16, qz,
                        out));
   }
   return finish_dequant(ctx, n);
