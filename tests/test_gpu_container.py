@@ -202,6 +202,15 @@ def test_column_map_edges(ctx, n):
         cdclq.dequantize_packed(ctx, qw, s16, qz, p32, ql.gbits, 128, "F32")
 
 
+@pytest.mark.parametrize("n,g,d_out", [(2048, 128, 4099), (2056, 8, 4097), (2047, 2047, 1025), (64, 16, 4095), (9, 8, 70)])
+def test_pack_runs_row_blocks(ctx, n, g, d_out):
+    """One and four rows per thread of the packing, with a last row block and a last run cut short."""
+    for wild in (False, True):
+        ql = _layer(n, g, d_out, n + d_out, wild=wild)
+        for a, b in zip(cdclq.pack_layer(ctx, ql), _oracle_pack(ql)):
+            _same_bits(a, b, f"pack n={n} d_out={d_out} wild={wild}")
+
+
 def test_device_entry_points_match_host(ctx):
     ql = _layer(4096, 128, 40, 9, gb=[4] * 32)
     d_out, n, g, ng = ql.d_out, ql.d_in, ql.group, ql.ngroups()
