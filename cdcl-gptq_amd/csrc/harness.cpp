@@ -333,10 +333,10 @@ int cdclq_proxy_loss_device(cdclq_ctx* ctx, const float* w_t, const float* w_hat
     HIPCK(pad_rows(ctx->st, (long)n, (int)n, ld, (int)ld, h, P<float>(ctx->mp)));
     h = P<float>(ctx->mp);
   }
-  CK(ensure(ctx, ctx->proxy_p, eval_partials(rows, (size_t)ld) * 8));
+  CK(ensure(ctx, ctx->proxy_p, eval_partials(rows, n) * 8));
   CK(ensure_pinned(ctx, 16));
   double* sums = static_cast<double*>(ctx->pin);
-  HIPCK(proxy_sum(ctx->st, (int)rows, (int)ld, (int)(direct ? n : (n + 31) & ~(size_t)31), P<float>(ctx->t1), ld, h,
+  HIPCK(proxy_sum(ctx->st, (int)rows, (int)n, (int)(direct ? n : (n + 31) & ~(size_t)31), P<float>(ctx->t1), ld, h,
                   ld, P<double>(ctx->proxy_p), sums));
   HIPCK(hipStreamSynchronize(ctx->st));
   *out = sums[0];

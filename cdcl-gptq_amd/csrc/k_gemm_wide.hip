@@ -206,8 +206,9 @@ __global__ __launch_bounds__(256, 2) void k_rel_err_tiles(int m, int n, int k, c
   reduce_pair(num, den, red, partial);
 }
 
-// engine::proxy_loss (src/engine.rs:808-815): the sum of e (e H) in f64; E m x k (row stride lde, its
-// first n columns the residual).
+// engine::proxy_loss (src/engine.rs:808-815): the sum of e (e H) in f64 over the residual's n columns; E
+// m x k (row stride lde) and H k x ldh are zero past them. Padding columns stay out of the sum: an infinite
+// residual times their zeros is NaN.
 __global__ __launch_bounds__(256, 2) void k_proxy_tiles(int m, int n, int k, const float* __restrict__ E, long lde,
                                                      const float* __restrict__ H, long ldh,
                                                      double* __restrict__ partial) {
@@ -218,14 +219,13 @@ __global__ __launch_bounds__(256, 2) void k_proxy_tiles(int m, int n, int k, con
   double s = 0.0;
   if (tile_of<Dense>(m, n, &r0, &cb)) {
     tile_v16f c[4];
-    chain_tile<Dense, false>(R, m, n, 0, k, E, lde, H, ldh, r0, cb, c);
+    chain_tile<Dense, false>(R, m, (int)ldh, 0, k, E, lde, H, ldh, r0, cb, c);
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       const int row = r0 + Dense::row(0, r, wv, lane), col = cb + Dense::col(0, lane);
-      if (row < m && col < n) {
 #pragma unroll
-        for (int b = 0; b < 4; ++b) s += (double)E[(long)row * lde + col + b] * (double)c[b][r];
-      }
+      for (int b = 0; b < 4; ++b)
+        if (row < m && col + b < n) s += (double)E[(long)row * lde + col + b] * (double)c[b][r];
     }
   }
   reduce_pair(s, 0.0, red, partial);

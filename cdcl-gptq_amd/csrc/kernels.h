@@ -151,7 +151,7 @@ hipError_t pad_rows(hipStream_t st, long rows, int n, long rows_out, int ld, con
 // sums of (o1 - o2)^2 and o1^2 over o1 = W X^T, o2 = W_hat Xt^T (W, W_hat m x k; X, Xt n x k)
 hipError_t rel_err_sums(hipStream_t st, int m, int n, int k, const float* W, const float* W_hat, long ldw,
                         const float* X, const float* Xt, long ldx, double* partial, double* out);
-// sum over m x n of e (E H) (E m x k, H k x n); out[1] = 0
+// sum over m x n of e (E H) (E m x k, H k x ldh, both zero in the columns past n); out[1] = 0
 hipError_t proxy_sum(hipStream_t st, int m, int n, int k, const float* E, long lde, const float* H, long ldh,
                      double* partial, double* out);
 hipError_t transpose_f32(hipStream_t st, int n, const float* src, float* dst);

@@ -93,6 +93,28 @@ def test_rel_err_and_proxy_loss_tile_edges(ctx, rows, n, t):
     assert abs(cdclq.proxy_loss(w, wq, rows, n, h, ctx) - O.proxy_loss(w, wq, h)) <= bound
 
 
+@pytest.mark.parametrize("n,off", [(5, 0), (33, 0), (333, 0), (352, 0), (352, 1)])
+def test_proxy_loss_of_an_infinite_residual(ctx, n, off):
+    """Padded widths, and an H off 16 bytes that is copied with padded rows: the padding takes no part in the
+    sum. With H and the residual positive, one infinite entry makes the loss infinite (the oracle's value);
+    a padding column would add 0 * (inf * 0) = NaN."""
+    rng = np.random.default_rng(n + off)
+    w = rng.uniform(1, 2, (3, n)).astype(np.float32)
+    wq = (w - 0.5).astype(np.float32)
+    w[1, n // 2] = np.inf
+    h = rng.uniform(1, 2, (n, n)).astype(np.float32)
+    assert O.proxy_loss(w, wq, h) == np.inf
+    dh = cdclq.DeviceArray.from_host(ctx, np.concatenate([np.zeros(off, np.float32), h.ravel()]))
+    dw, dq = (cdclq.DeviceArray.from_host(ctx, a) for a in (w, wq))
+    out = cdclq.C.c_double()
+    print(f"[bench] proxy loss inf n={n} off={off}", flush=True)
+    ctx.check(cdclq.lib().cdclq_proxy_loss_device(ctx.ptr, dw.ptr, dq.ptr, 3, n, dh.ptr.value + 4 * off,
+                                                  cdclq.C.byref(out)))
+    assert out.value == np.inf
+    for a in (dw, dq, dh):
+        a.free()
+
+
 def test_bench_run_reproduces_the_readme_table(ctx):
     """`cdclq bench --rows 512 --cols 2048 --tokens 16384 --test-tokens 4096` (3 bit, group 128):
     every held-out error and percentage the README prints (README.md:207-219)."""
