@@ -10,6 +10,8 @@
 // The panel solve and the blocks' inverse give a row several lanes (its columns interleaved over
 // them): column t is finalised at step t and immediately subtracted from every later column, which
 // performs the reference's per-element subtraction sequence in the same order.
+#include <algorithm>
+
 #include "cdclq_dev.h"
 #include "kernels.h"
 
@@ -22,24 +24,26 @@ constexpr int NBC = 96;  // src/linalg.rs:202, :285
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 // hp = perm(H) in f64, dead diagonal -> 1, + damp on the diagonal; h32 = (f32)hp; a = flip(hp).
-// h32 is ld x ld, zero past n.
+// h32 is ld x ld, zero past n. Grid-stride: the padded matrix of n = 65535 has 2^32 elements, one
+// more than a launch may have work-items.
 __global__ __launch_bounds__(256) void k_build_flipped(int n, int ld, const float* __restrict__ h,
                                                        const uint32_t* __restrict__ perm, double damp_val,
                                                        double* __restrict__ a, float* __restrict__ h32) {
-  const long idx = (long)blockIdx.x * 256 + threadIdx.x;
-  if (idx >= (long)ld * ld) return;
-  const int p = (int)(idx / ld), q = (int)(idx % ld);
-  if (p >= n || q >= n) {
-    h32[idx] = 0.0f;
-    return;
+  const long count = (long)ld * ld;
+  for (long idx = (long)blockIdx.x * 256 + threadIdx.x; idx < count; idx += (long)gridDim.x * 256) {
+    const int p = (int)(idx / ld), q = (int)(idx % ld);
+    if (p >= n || q >= n) {
+      h32[idx] = 0.0f;
+      continue;
+    }
+    double v = (double)h[(long)perm[p] * n + perm[q]];
+    if (p == q) {
+      if (v == 0.0) v = 1.0;
+      v = v + damp_val;
+    }
+    h32[idx] = (float)v;
+    a[(long)(n - 1 - p) * n + (n - 1 - q)] = v;
   }
-  double v = (double)h[(long)perm[p] * n + perm[q]];
-  if (p == q) {
-    if (v == 0.0) v = 1.0;
-    v = v + damp_val;
-  }
-  h32[idx] = (float)v;
-  a[(long)(n - 1 - p) * n + (n - 1 - q)] = v;
 }
 
 __global__ __launch_bounds__(256) void k_build_flipped_f64(int n, const double* __restrict__ h, double* __restrict__ a) {
@@ -331,7 +335,8 @@ inline unsigned nblk(long count) { return (unsigned)((count + 255) / 256); }
 
 hipError_t build_flipped(hipStream_t st, int n, int ld, const float* h, const uint32_t* perm, double damp_val,
                          double* a, float* h32) {
-  hipLaunchKernelGGL(k_build_flipped, dim3(nblk((long)ld * ld)), dim3(256), 0, st, n, ld, h, perm, damp_val, a, h32);
+  const unsigned grid = (unsigned)std::min<long>(((long)ld * ld + 255) / 256, 1L << 20);
+  hipLaunchKernelGGL(k_build_flipped, dim3(grid), dim3(256), 0, st, n, ld, h, perm, damp_val, a, h32);
   return hipGetLastError();
 }
 

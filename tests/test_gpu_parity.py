@@ -292,6 +292,29 @@ def test_upper_chol_block_edges_bitexact(ctx, n, sparse):
     assert np.array_equal(ug.view(np.uint32), uo.view(np.uint32)), f"{(ug != uo).sum()} U entries differ"
 
 
+def test_prepare_widest_layer():
+    """d_in = 65535, the widest layer accepted: its padded Hessian has 2^32 elements. A Hessian with a negative
+    diagonal ends in the factorisation's own error, after the launches that build its operands. (About
+    120 GB of device memory, released with the context.)"""
+    n, L = 65535, cdclq.lib()
+    c = cdclq.Context(0)
+    h, w = cdclq.C.c_void_p(), cdclq.C.c_void_p()
+    try:
+        c.check(L.cdclq_device_alloc(c.ptr, n * 4, cdclq.C.byref(w)))
+        c.check(L.cdclq_device_alloc(c.ptr, n * n * 4, cdclq.C.byref(h)))
+        c.check(L.cdclq_memset_device(c.ptr, w, 0, n * 4))
+        c.check(L.cdclq_memset_device(c.ptr, h, 0xBF, n * n * 4))  # every entry -1.498
+        print(f"[prepare] n={n}", flush=True)
+        rc = L.cdclq_prepare_layer_device(c.ptr, w, 1, n, h, b"wide", cdclq.C.byref(cdclq.Config()._c()))
+        msg = L.cdclq_last_error(c.ptr).decode()
+        assert rc == 2 and "not positive definite (pivot 0 " in msg, (rc, msg)
+    finally:
+        for p in (w, h):
+            if p:
+                L.cdclq_device_free(c.ptr, p)
+        c.close()
+
+
 def _spd_fast(n, seed):
     """M M^T / n + I with M n x (n + 8) from numpy's generator (rand_spd's per-draw loop is slow at
     this size); any SPD input serves for bit parity."""
