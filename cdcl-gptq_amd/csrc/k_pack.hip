@@ -399,7 +399,8 @@ __global__ __launch_bounds__(256) void k_pack_runs(long d_out, int n, int rb, in
                                                    const uint32_t* __restrict__ rdesc, uint8_t* __restrict__ qw,
                                                    uint32_t* __restrict__ spill, uint32_t epoch) {
   const int k = (int)(blockIdx.y << lx) + (int)(threadIdx.x & ((1u << lx) - 1u));
-  const long r0 = ((long)blockIdx.x * (256 >> lx) + (threadIdx.x >> lx)) * R;
+  const long blk = (long)blockIdx.z * gridDim.x + blockIdx.x;
+  const long r0 = (blk * (256 >> lx) + (threadIdx.x >> lx)) * R;
   if (k >= runs || r0 >= d_out) return;
   const int j0 = 8 * k, m = min(8, n - j0);
   const int nr = (int)min((long)R, d_out - r0);
@@ -486,15 +487,14 @@ hipError_t pack_runs(hipStream_t st, long d_out, int n, int rb, const uint8_t* c
   // (kernel at 2048 x 2048 3.2 us with one row and 3.6 with four, 4001 x 1350 6.0 and 7.6, 32 x 16384
   // 2.3 and 2.9; at 2^20 runs, 4096 x 2048, four rows take
   // 4.6 us where one row with the division took 5.4).
-  if (n % 8 == 0 && d_out * runs >= (1L << 20)) {
-    const long per = 4L * (256 >> lx);
-    hipLaunchKernelGGL(k_pack_runs<4>, dim3((unsigned)((d_out + per - 1) / per), gy), dim3(256), 0, st, d_out, n, rb,
-                       runs, lx, codes, rdesc, qw, spill, epoch);
-  } else {
-    const long per = 256 >> lx;
-    hipLaunchKernelGGL(k_pack_runs<1>, dim3((unsigned)((d_out + per - 1) / per), gy), dim3(256), 0, st, d_out, n, rb,
-                       runs, lx, codes, rdesc, qw, spill, epoch);
-  }
+  const bool four = n % 8 == 0 && d_out * runs >= (1L << 20);
+  const long per = (four ? 4L : 1L) * (256 >> lx), blocks = (d_out + per - 1) / per;
+  const long gx = std::min<long>(blocks, 1L << 20);  // a launch takes fewer than 2^32 work-items along x
+  const dim3 grid((unsigned)gx, gy, (unsigned)((blocks + gx - 1) / gx));
+  if (four)
+    hipLaunchKernelGGL(k_pack_runs<4>, grid, dim3(256), 0, st, d_out, n, rb, runs, lx, codes, rdesc, qw, spill, epoch);
+  else
+    hipLaunchKernelGGL(k_pack_runs<1>, grid, dim3(256), 0, st, d_out, n, rb, runs, lx, codes, rdesc, qw, spill, epoch);
   return hipGetLastError();
 }
 

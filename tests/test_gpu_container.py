@@ -211,6 +211,38 @@ def test_pack_runs_row_blocks(ctx, n, g, d_out):
             _same_bits(a, b, f"pack n={n} d_out={d_out} wild={wild}")
 
 
+def test_pack_more_rows_than_work_items_along_x():
+    """2^24 + 5 rows of 129 runs (17 GB of codes): a workgroup per row along x alone would be a launch of 2^32
+    work-items. The first and last rows are compared."""
+    c, L = cdclq.Context(0), cdclq.lib()
+    d_out, n, k = (1 << 24) + 5, 1025, 300
+    rb, rng = cdclq.row_bytes(n, n, [1]), np.random.default_rng(3)
+    size = dict(codes=d_out * n, scales=4 * d_out, zeros=4 * d_out, perm=4 * n, qw=d_out * rb, s16=2 * d_out, qz=d_out,
+                p32=4 * n)
+    buf = {name: cdclq.C.c_void_p() for name in size}
+    try:
+        for name, p in buf.items():
+            c.check(L.cdclq_device_alloc(c.ptr, size[name], cdclq.C.byref(p)))
+            c.check(L.cdclq_memset_device(c.ptr, p, 0, size[name]))
+        ends = {0: rng.integers(0, 2, (k, n), dtype=np.uint8), d_out - k: rng.integers(0, 2, (k, n), dtype=np.uint8)}
+        for r, a in ends.items():
+            c.check(L.cdclq_memcpy_h2d(c.ptr, buf["codes"].value + r * n, a.ctypes.data, a.nbytes))
+        gb = np.ones(1, np.uint8)
+        print(f"[container] pack d_out={d_out} n={n}", flush=True)
+        c.check(L.cdclq_pack_layer_device(c.ptr, d_out, n, n, gb.ctypes.data, 1, buf["codes"], buf["scales"],
+                                          buf["zeros"], buf["perm"], buf["qw"], size["qw"], buf["s16"], buf["qz"],
+                                          buf["p32"]))
+        for r, a in ends.items():
+            got = np.empty((k, rb), np.uint8)
+            c.check(L.cdclq_memcpy_d2h(c.ptr, got.ctypes.data, buf["qw"].value + r * rb, got.nbytes))
+            assert np.array_equal(got, np.packbits(a, axis=1, bitorder="little")), f"rows from {r}"
+    finally:
+        for p in buf.values():
+            if p:
+                L.cdclq_device_free(c.ptr, p)
+        c.close()
+
+
 def test_device_entry_points_match_host(ctx):
     ql = _layer(4096, 128, 40, 9, gb=[4] * 32)
     d_out, n, g, ng = ql.d_out, ql.d_in, ql.group, ql.ngroups()
