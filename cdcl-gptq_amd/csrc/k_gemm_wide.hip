@@ -296,6 +296,9 @@ bool chain_gemm_tiles_ok(int m, int n, int k, const float* A, long lda, const fl
          (long)m * lda < (1L << 31) && (long)k * ldb < (1L << 31);
 }
 
+// The most workgroups of 256 a launch may have: 2^32 work-items wrap to a smaller launch without an error.
+constexpr long MAX_GRID = (1L << 24) - 1;
+
 // workgroups over an m x n output: every XCD gets the same number of block slots
 template <class T>
 static long tile_grid(long m, long n) {
@@ -319,7 +322,7 @@ hipError_t pad_rows(hipStream_t st, long rows, int n, long rows_out, int ld, con
 hipError_t rel_err_sums(hipStream_t st, int m, int n, int k, const float* W, const float* W_hat, long ldw,
                         const float* X, const float* Xt, long ldx, double* partial, double* out) {
   const long grid = tile_grid<DenseT>(m, n);
-  if (grid > 0x7fffffffL) return hipErrorInvalidValue;
+  if (grid > MAX_GRID) return hipErrorInvalidValue;
   hipLaunchKernelGGL(k_rel_err_tiles, dim3((unsigned)grid), dim3(256), 0, st, m, n, k, W, W_hat, ldw, X, Xt, ldx,
                      partial);
   hipError_t err = hipGetLastError();
@@ -331,7 +334,7 @@ hipError_t rel_err_sums(hipStream_t st, int m, int n, int k, const float* W, con
 hipError_t proxy_sum(hipStream_t st, int m, int n, int k, const float* E, long lde, const float* H, long ldh,
                      double* partial, double* out) {
   const long grid = tile_grid<Dense>(m, n);
-  if (grid > 0x7fffffffL) return hipErrorInvalidValue;
+  if (grid > MAX_GRID) return hipErrorInvalidValue;
   hipLaunchKernelGGL(k_proxy_tiles, dim3((unsigned)grid), dim3(256), 0, st, m, n, k, E, lde, H, ldh, partial);
   hipError_t err = hipGetLastError();
   if (err != hipSuccess) return err;
@@ -342,7 +345,7 @@ hipError_t proxy_sum(hipStream_t st, int m, int n, int k, const float* E, long l
 hipError_t chain_gemm_tiles(hipStream_t st, int m, int n, int k, const float* A, long lda, const float* B, long ldb,
                             float* C, long ldc, int tri) {
   const long grid = tile_grid<Dense>(m, n);
-  if (grid > 0x7fffffffL) return hipErrorInvalidValue;
+  if (grid > MAX_GRID) return hipErrorInvalidValue;
   if (tri == 1)
     hipLaunchKernelGGL(k_chain_gemm_tiles<1>, dim3((unsigned)grid), dim3(256), 0, st, m, n, k, A, lda, B, ldb, C, ldc);
   else if (tri == 2)

@@ -115,6 +115,20 @@ def test_proxy_loss_of_an_infinite_residual(ctx, n, off):
         a.free()
 
 
+def test_rel_err_refuses_more_tiles_than_a_launch_takes(ctx):
+    """2^20 + 1 rows by 131136 tokens are over 2^24 tiles: an error, not the sum of a wrapped launch."""
+    rows, n, t = (1 << 20) + 1, 32, 131136
+    L, out = cdclq.lib(), cdclq.C.c_double(-1.0)
+    w, x = (cdclq.DeviceArray(ctx, (r, n), np.float32) for r in (rows, t))
+    for a in (w, x):
+        a.zero()
+    print(f"[bench] rel_err rows={rows} t={t}", flush=True)
+    with pytest.raises(cdclq.CdclqError):
+        ctx.check(L.cdclq_rel_err_device(ctx.ptr, w.ptr, w.ptr, x.ptr, x.ptr, rows, n, t, cdclq.C.byref(out)))
+    for a in (w, x):
+        a.free()
+
+
 def test_bench_run_reproduces_the_readme_table(ctx):
     """`cdclq bench --rows 512 --cols 2048 --tokens 16384 --test-tokens 4096` (3 bit, group 128):
     every held-out error and percentage the README prints (README.md:207-219)."""
