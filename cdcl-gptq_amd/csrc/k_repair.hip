@@ -19,6 +19,7 @@
 #include "cdclq_dev.h"
 #include "kernels.h"
 #include "mfma_tile.h"
+#include "repair_rule.h"
 
 namespace cdclq {
 namespace {
@@ -1504,15 +1505,11 @@ hipError_t panel_gemm(hipStream_t st, int m, int wd, int k, const float* A, long
     int cus = 0;
     const hipError_t err = device_cus(&cus);
     if (err != hipSuccess) return err;
-    // 128 x 128 tiles from 2.5 a CU (2048 x 5632, 2.6 a CU: 58.1 us against 61.4 on 128 x 64; 5632 x
-    // 2048, 2.4 a CU: 57.4 against 52.0), 64 x 64 ones where 128 x 64 tiles would leave CUs without one
-    // (1001 x 1350: 14.2 against 14.8 us)
-    const long units = ntiles * np;
-    if (2 * units * ((wd + 127) / 128) >= 5L * cus)
-      return grad_launch<GradM, 2>(st, m, wd, k, A, lda, B, ldb, P, rtiles, ntiles, np, skip);
-    if (units * ((wd + 63) / 64) >= cus)
-      return grad_launch<GradD, 2>(st, m, wd, k, A, lda, B, ldb, P, rtiles, ntiles, np, skip);
-    return grad_launch<GradS, 3>(st, m, wd, k, A, lda, B, ldb, P, rtiles, ntiles, np, skip);
+    switch (grad_tile(ntiles * np, wd, cus)) {
+      case GRAD_128x128: return grad_launch<GradM, 2>(st, m, wd, k, A, lda, B, ldb, P, rtiles, ntiles, np, skip);
+      case GRAD_128x64: return grad_launch<GradD, 2>(st, m, wd, k, A, lda, B, ldb, P, rtiles, ntiles, np, skip);
+      default: return grad_launch<GradS, 3>(st, m, wd, k, A, lda, B, ldb, P, rtiles, ntiles, np, skip);
+    }
   }
   if (skip >= 0) return hipErrorInvalidValue;
   // groups or sub-blocks that start or end off a multiple of 4 columns
