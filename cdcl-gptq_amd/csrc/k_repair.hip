@@ -324,6 +324,7 @@ __global__ __launch_bounds__(T::THREADS) void k_grad(int m, int wd, int k, const
 typedef MfmaTile<4, 1, 1, 4> GradM;  // 128 x 128, ring of two, 2 workgroups
 typedef MfmaTile<4, 1, 1, 2> GradD;  // 128 x 64, ring of two, 3 workgroups
 typedef MfmaTile<2, 2, 1, 1> GradS;  // 64 x 64, ring of three, 3 workgroups
+typedef MfmaTile<4, 1, 1, 1> GradN;  // 128 x 32, ring of two, 4 workgroups
 
 // The GPTQ lazy trailing update C = C - A B (src/engine.rs:452-471), one chain per kfold steps of k
 // (kfold <= 256: one KC panel), each folded straight into the C values held in registers in k order,
@@ -1507,6 +1508,7 @@ hipError_t panel_gemm(hipStream_t st, int m, int wd, int k, const float* A, long
     if (err != hipSuccess) return err;
     switch (grad_tile(ntiles * np, wd, cus)) {
       case GRAD_128x128: return grad_launch<GradM, 2>(st, m, wd, k, A, lda, B, ldb, P, rtiles, ntiles, np, skip);
+      case GRAD_128x32: return grad_launch<GradN, 2>(st, m, wd, k, A, lda, B, ldb, P, rtiles, ntiles, np, skip);
       case GRAD_128x64: return grad_launch<GradD, 2>(st, m, wd, k, A, lda, B, ldb, P, rtiles, ntiles, np, skip);
       default: return grad_launch<GradS, 3>(st, m, wd, k, A, lda, B, ldb, P, rtiles, ntiles, np, skip);
     }

@@ -451,6 +451,16 @@ def test_quantize_wide_gradient_tiles(ctx):
                 label="wide gradient tiles")
 
 
+@pytest.mark.parametrize("sub_block", [4, 24, 32, 48])
+def test_quantize_narrow_gradient_tiles(ctx, sub_block):
+    """Descent gradients of 32 columns and fewer (tiles of 128 x 32) and of 48 (128 x 64) with a tile for every
+    CU: 16500 rows x 300 columns are 129 row tiles (a ragged last one) x 2 panels; widths off a multiple of 32
+    and a ragged last sub-block."""
+    w, x, h, _ = synth_layer(53, 16500, 300, 700)
+    assert_same(*run_both(ctx, w, h, bits=3, group=64, block=128, act_order=True, passes=2, sub_block=sub_block,
+                          refit_scales=False, row_chunk=64), label=f"narrow gradient {sub_block}")
+
+
 @pytest.mark.parametrize("d_out,n,group", [
     (33, 40, 0), (70, 100, 0),                       # one group, one panel
     (40, 300, 8), (1025, 257, 16), (65, 511, 32),    # several groups per 64-column piece, ragged panels

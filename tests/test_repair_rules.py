@@ -29,11 +29,13 @@ def rules(tmp_path_factory):
 @pytest.mark.parametrize("wd", [4, 8, 16, 32, 48, 60, 64, 68, 96, 100, 128, 192, 196, 256, 320, 512, 1000, 1024])
 def test_gradient_tile_computes_few_spare_columns(rules, wd):
     """The 128-column tile computes at most 1/19 more columns than 64-column ones would, and is still taken
-    for widths that it divides once it fills the device."""
-    cols = {0: 128, 1: 64, 2: 64}
+    for widths that it divides once it fills the device; 32 columns and fewer take the 32-column tile there."""
+    cols = {0: 128, 1: 64, 2: 64, 3: 32}
     least = (wd + 63) // 64 * 64
     for units in (1, 255, 256, 640, 1792, 100000):
         t = rules.r_grad_tile(units, wd, 256)
         assert -(-wd // cols[t]) * cols[t] * 19 <= least * 20, (units, t)
         if wd % 128 == 0 and 2 * units * (wd // 128) >= 5 * 256:
             assert t == 0
+        if units >= 256 and wd <= 64:
+            assert t == (3 if wd <= 32 else 1)
