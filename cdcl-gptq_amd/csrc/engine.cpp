@@ -21,6 +21,7 @@
 #include "cdclq_dev.h"
 #include "ctx.h"
 #include "kernels.h"
+#include "repair_rule.h"
 
 namespace {
 
@@ -495,8 +496,10 @@ int quantize_device(cdclq_ctx* ctx, const float* w, size_t d_out_, size_t n_, co
     CK(ensure(ctx, ctx->ebuf, (size_t)d_out * lde * 4));
     eb = P<float>(ctx->ebuf);
     HIPCK(residual(st, d_out, n, lde, wp, wq, eb));
-    // steps whose groups / sub-blocks lie inside the KC panels run one panel per launch
-    const bool rpanel = do_refit && refit_panel_ok(n, g), cpanel = do_cd && cd_panel_ok(n, sbw);
+    // steps whose groups / sub-blocks lie inside the KC panels run one panel per launch (repair_rule.h)
+    int cus = 0;
+    HIPCK(device_cus(&cus));
+    const bool rpanel = do_refit && refit_panel_ok(n, g, d_out, cus), cpanel = do_cd && cd_panel_ok(n, sbw);
     const int wdmax = std::max(do_cd && !cpanel ? sbw : 1, do_refit && !rpanel ? g : 1);
     const int wpart = std::max(wdmax, np > 1 && (rpanel || cpanel) ? std::min(lde, CDCLQ_KC) : 1);
     CK(ensure(ctx, ctx->part, panel_partials_elems(d_out, wpart, n) * 4));

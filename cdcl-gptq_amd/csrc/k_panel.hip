@@ -568,7 +568,6 @@ int panel_rows(int rows, int cus) { return rows <= 4 * cus ? 4 : (rows <= 8 * cu
 
 }  // namespace
 
-bool refit_panel_ok(int n, int g) { return g <= 128 && (g >= n || g == 128 || (g >= 16 && 64 % g == 0)); }
 bool cd_panel_ok(int n, int sbw) { return sbw == PW || (sbw >= n && n <= PW); }
 
 hipError_t refit_panel(hipStream_t st, const RefitPanelArgs& a) {

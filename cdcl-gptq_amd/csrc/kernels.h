@@ -205,7 +205,6 @@ struct CdPanelArgs {
   unsigned long long* mid;
   uint32_t* evals;
 };
-bool refit_panel_ok(int n, int g);
 bool cd_panel_ok(int n, int sbw);
 hipError_t refit_panel(hipStream_t st, const RefitPanelArgs& a);
 hipError_t cd_panel(hipStream_t st, const CdPanelArgs& a);

@@ -20,4 +20,18 @@ inline GradTile grad_tile(long units, int wd, int cus) {
   return wd <= 32 ? GRAD_128x32 : GRAD_128x64;
 }
 
+// Whether the refit of `rows` rows in groups of g runs a KC panel of groups per launch (k_panel.hip,
+// k_refit_panel) and not a launch pair per group. The groups have to lie inside the panels: 16, 32, 64 or 128
+// columns, or one group of all n <= 128. A panel launch keeps one workgroup of at most 16 rows a CU where the
+// per-group refit keeps two of up to 64, so what it saves in launches it loses again in rounds: groups of
+// two 64-column pieces from the third round on (refit of one pass and the last, groups of 128: 8192 x
+// 2048 3.11 against 3.15 ms, 12288 x 2048 4.46 and 4.10, 14336 x 4096 17.5 and 15.5, 131072 x 512 6.67 and 4.53),
+// one group alone, which saves a single launch, from the fifth (131072 x 64 0.58 and 0.51; 16384 x 64 0.157 and
+// 0.161); several groups of 64 and less to a panel never (131072 x 256, groups of 16, 7.31 and 7.44).
+inline bool refit_panel_ok(int n, int g, int rows, int cus) {
+  if (!(g <= 128 && (g >= n || g == 128 || (g >= 16 && 64 % g == 0)))) return false;
+  if (g > 64) return rows <= 32L * cus;
+  return g < n || rows <= 64L * cus;
+}
+
 }  // namespace cdclq

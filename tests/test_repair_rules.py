@@ -11,6 +11,7 @@ SHIM = """
 using namespace cdclq;
 extern "C" {
 int r_grad_tile(long units, int wd, int cus) { return (int)grad_tile(units, wd, cus); }
+int r_refit_panel_ok(int n, int g, int rows, int cus) { return refit_panel_ok(n, g, rows, cus); }
 }
 """
 
@@ -39,3 +40,15 @@ def test_gradient_tile_computes_few_spare_columns(rules, wd):
             assert t == 0
         if units >= 256 and wd <= 64:
             assert t == (3 if wd <= 32 else 1)
+
+
+@pytest.mark.parametrize("n,g,most", [  # the most rows on 256 CUs; None: any number
+    (2048, 128, 8192), (128, 128, 8192), (100, 100, 8192), (65, 65, 8192),   # two pieces to a group
+    (64, 64, 16384), (20, 20, 16384),                                        # one group, one piece
+    (65, 64, None), (2048, 64, None), (2048, 32, None), (300, 16, None),     # groups inside a piece
+    (2048, 8, 0), (2048, 96, 0), (2048, 256, 0), (300, 300, 0), (2048, 24, 0),
+])
+def test_refit_by_panels(rules, n, g, most):
+    """Groups that fit the panels' pieces take the panel launch while their rows are few rounds of it."""
+    for rows in (1, 4096, 8192, 8193, 16384, 16385, 1 << 20):
+        assert rules.r_refit_panel_ok(n, g, rows, 256) == (most is None or rows <= most), rows
