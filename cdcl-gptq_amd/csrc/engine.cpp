@@ -499,7 +499,7 @@ int quantize_device(cdclq_ctx* ctx, const float* w, size_t d_out_, size_t n_, co
     // steps whose groups / sub-blocks lie inside the KC panels run one panel per launch (repair_rule.h)
     int cus = 0;
     HIPCK(device_cus(&cus));
-    const bool rpanel = do_refit && refit_panel_ok(n, g, d_out, cus), cpanel = do_cd && cd_panel_ok(n, sbw);
+    const bool rpanel = do_refit && refit_panel_ok(n, g, d_out, cus), cpanel = do_cd && cd_panel_ok(n, sbw, d_out, cus);
     const int wdmax = std::max(do_cd && !cpanel ? sbw : 1, do_refit && !rpanel ? g : 1);
     const int wpart = std::max(wdmax, np > 1 && (rpanel || cpanel) ? std::min(lde, CDCLQ_KC) : 1);
     CK(ensure(ctx, ctx->part, panel_partials_elems(d_out, wpart, n) * 4));
@@ -527,17 +527,19 @@ int quantize_device(cdclq_ctx* ctx, const float* w, size_t d_out_, size_t n_, co
     std::vector<double> prev(nchunks, 0.0);
     std::vector<uint64_t> upd(nchunks);
     // The gradient GEMM runs only over the 128-row tiles that hold rows of a chunk still being
-    // repaired: list 0 for the refit steps (active chunks), list 1 + s for the descent's step s, a
-    // sub-block or a panel of spl sub-blocks (active chunks that selected one of them). A null list
-    // means every tile (the final refit).
+    // repaired: list 0 for the refit steps (active chunks), one list per step of the descent, a sub-block
+    // or a panel of them (active chunks that selected one of them). A null list means every tile (the
+    // final refit).
     const int rt = panel_row_tile(), ntile = (d_out + rt - 1) / rt;
-    const int spl = cpanel ? CDCLQ_KC / 64 : 1, ncd = (n_sb + spl - 1) / spl;
-    auto selected = [&](int c, int s) {  // chunk c takes part in descent step s
-      bool any = false;
-      for (int t = s * spl; t < std::min((s + 1) * spl, n_sb) && !any; ++t) any = sel[(size_t)c * n_sb + t];
-      return act[c] && any;
+    struct CdStep {
+      bool panel;
+      int s;     // sub-block, or panel
+      int list;  // its tiles
+      int cnt;
     };
-    std::vector<int> tl((size_t)(1 + ncd) * ntile), tcnt(1 + ncd);
+    std::vector<CdStep> steps;
+    std::vector<int> tl((size_t)(1 + n_sb) * ntile), both;
+    int nl = 0, nt_act = 0;  // lists in use, tiles of list 0
     const size_t apad = ((size_t)nchunks + 15) / 16 * 16, up_bytes = apad + tl.size() * sizeof(int);
     CK(ensure(ctx, ctx->rtiles_d, up_bytes));
     uint8_t* active = P<uint8_t>(ctx->rtiles_d);
@@ -547,8 +549,9 @@ int quantize_device(cdclq_ctx* ctx, const float* w, size_t d_out_, size_t n_, co
     char* pin_down = pin_up + up_bytes;
     auto upload_pass = [&]() -> int {  // the previous upload has finished: every pass ends in a sync
       std::memcpy(pin_up, act.data(), nchunks);
-      std::memcpy(pin_up + apad, tl.data(), tl.size() * sizeof(int));
-      HIPCK(hipMemcpyAsync(ctx->rtiles_d.p, pin_up, up_bytes, hipMemcpyHostToDevice, st));
+      const size_t lists = (size_t)nl * ntile * sizeof(int);
+      std::memcpy(pin_up + apad, tl.data(), lists);
+      HIPCK(hipMemcpyAsync(ctx->rtiles_d.p, pin_up, apad + lists, hipMemcpyHostToDevice, st));
       return CDCLQ_OK;
     };
     auto download_pass = [&]() -> int {
@@ -559,16 +562,46 @@ int quantize_device(cdclq_ctx* ctx, const float* w, size_t d_out_, size_t n_, co
       return CDCLQ_OK;
     };
     auto build_tiles = [&]() -> int {
-      for (int l = 0; l <= ncd; ++l) {
-        int cnt = 0;
+      // the tiles of chunks that take part (take(chunk)) to tl's next list
+      auto add_list = [&](auto take) -> int {
+        int cnt = 0, *out = tl.data() + (size_t)nl * ntile;
         for (int t = 0; t < ntile; ++t) {
           const int c_lo = (t * rt) / rc, c_hi = (std::min((t + 1) * rt, d_out) - 1) / rc;
           bool need = false;
-          for (int c = c_lo; c <= c_hi && !need; ++c)
-            need = l == 0 ? act[c] != 0 : selected(c, l - 1);
-          if (need) tl[(size_t)l * ntile + cnt++] = t;
+          for (int c = c_lo; c <= c_hi && !need; ++c) need = take(c);
+          if (need) out[cnt++] = t;
         }
-        tcnt[l] = cnt;
+        ++nl;
+        return cnt;
+      };
+      nl = 0;
+      steps.clear();
+      nt_act = add_list([&](int c) { return act[c] != 0; });
+      const int per = cpanel ? CDCLQ_KC / 64 : 1;
+      for (int s0 = 0; do_cd && s0 < n_sb; s0 += per) {
+        const int l0 = nl, nsub = std::min(per, n_sb - s0);
+        const size_t st0 = steps.size();
+        int cnt[CDCLQ_KC / 64];
+        for (int i = 0; i < nsub; ++i) {
+          cnt[i] = add_list([&](int c) { return act[c] && sel[(size_t)c * n_sb + s0 + i]; });
+          if (cnt[i])
+            steps.push_back({false, s0 + i, nl - 1, cnt[i]});
+          else
+            --nl;
+        }
+        if (!cpanel || nl == l0) continue;
+        both.clear();
+        for (size_t k = st0; k < steps.size(); ++k) {
+          const int* l = tl.data() + (size_t)steps[k].list * ntile;
+          const auto mid = both.insert(both.end(), l, l + steps[k].cnt);
+          std::inplace_merge(both.begin(), mid, both.end());
+          both.erase(std::unique(both.begin(), both.end()), both.end());
+        }
+        if (!cd_panel_pays(cnt, nsub, (int)both.size(), np, d_out, cus)) continue;
+        steps.resize(st0);
+        std::copy(both.begin(), both.end(), tl.begin() + (size_t)l0 * ntile);
+        nl = l0 + 1;
+        steps.push_back({true, s0 / per, l0, (int)both.size()});
       }
       return upload_pass();
     };
@@ -577,7 +610,7 @@ int quantize_device(cdclq_ctx* ctx, const float* w, size_t d_out_, size_t n_, co
     auto refit_all = [&]() -> int {
       HIPCK(hipMemsetAsync(rcnt, 0, (size_t)ng * d_out * 4, st));
       const int* tl0 = all_tiles ? nullptr : rtiles;
-      const int nt0 = all_tiles ? ntile : tcnt[0];
+      const int nt0 = all_tiles ? ntile : nt_act;
       for (int q = 0; rpanel && q < np; ++q) {
         const int c0 = q * CDCLQ_KC, wdp = std::min(lde - c0, CDCLQ_KC);
         if (np > 1)
@@ -605,13 +638,13 @@ int quantize_device(cdclq_ctx* ctx, const float* w, size_t d_out_, size_t n_, co
       if (do_refit) CK(refit_all());
       if (do_cd) {
         HIPCK(hipMemsetAsync(ccnt, 0, (size_t)n_sb * d_out * 4, st));
-        for (int s = 0; s < ncd; ++s) {
-          if (tcnt[1 + s] == 0) continue;
-          const int* tl_s = rtiles + (size_t)(1 + s) * ntile;
-          if (cpanel) {
+        for (const CdStep& step : steps) {
+          const int s = step.s;
+          const int* tl_s = rtiles + (size_t)step.list * ntile;
+          if (step.panel) {
             const int c0 = s * CDCLQ_KC, wdp = std::min(lde - c0, CDCLQ_KC);
             if (np > 1)
-              HIPCK(panel_gemm(st, d_out, wdp, kp, eb, lde, H32 + c0, lde, P<float>(ctx->part), tl_s, tcnt[1 + s], s));
+              HIPCK(panel_gemm(st, d_out, wdp, kp, eb, lde, H32 + c0, lde, P<float>(ctx->part), tl_s, step.cnt, s));
             HIPCK(cd_panel(st, CdPanelArgs{d_out, n, lde, ng, g, s, n_sb, rc, (int)cfg->cd_sweeps, cap, np, wdp,
                                            P<float>(ctx->part), H32, P<uint8_t>(ctx->gbits_d), scales, zeros, codes,
                                            wq, eb, active, P<uint8_t>(ctx->sel_d), clog, ccnt, mid, cd_evals}));
@@ -621,9 +654,9 @@ int quantize_device(cdclq_ctx* ctx, const float* w, size_t d_out_, size_t n_, co
           // the descent kernel folds the per-panel chains itself where it can (one launch less)
           const bool fused = cd_folds_chains(wd);
           if (fused)
-            HIPCK(panel_gemm(st, d_out, wd, kp, eb, lde, H32 + c0, lde, P<float>(ctx->part), tl_s, tcnt[1 + s]));
+            HIPCK(panel_gemm(st, d_out, wd, kp, eb, lde, H32 + c0, lde, P<float>(ctx->part), tl_s, step.cnt));
           else
-            CK(grad_gemm(ctx, d_out, n, c0, wd, eb, H32, tl_s, tcnt[1 + s]));
+            CK(grad_gemm(ctx, d_out, n, c0, wd, eb, H32, tl_s, step.cnt));
           HIPCK(cd_subblock(st, d_out, n, lde, ng, g, c0, wd, s, n_sb, rc, (int)cfg->cd_sweeps, P<float>(ctx->G), H32,
                             P<uint8_t>(ctx->gbits_d), scales, zeros, codes, wq, eb, active,
                             P<uint8_t>(ctx->sel_d), clog + (size_t)s * d_out * cap, ccnt + (size_t)s * d_out, cap,

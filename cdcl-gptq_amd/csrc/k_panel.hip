@@ -568,8 +568,6 @@ int panel_rows(int rows, int cus) { return rows <= 4 * cus ? 4 : (rows <= 8 * cu
 
 }  // namespace
 
-bool cd_panel_ok(int n, int sbw) { return sbw == PW || (sbw >= n && n <= PW); }
-
 hipError_t refit_panel(hipStream_t st, const RefitPanelArgs& a) {
   int cus = 0;
   const hipError_t err = device_cus(&cus);

@@ -173,8 +173,8 @@ hipError_t cd_subblock(hipStream_t st, int rows, int n, int ld, int ng, int g, i
                        uint32_t* evals, const float* P = nullptr, int np = 0);
 // ---- k_panel.hip: the refit groups / the 64-column descent sub-blocks of KC panel q, one after
 // another in one launch. P holds the other np - 1 panels' chains over the panel's wdp columns
-// (panel_gemm with skip = q; unread when np == 1). The _ok tests say
-// which group and sub-block widths it takes (else one refit_group / cd_subblock per step).
+// (panel_gemm with skip = q; unread when np == 1). repair_rule.h says which widths and sizes take them
+// (else one refit_group / cd_subblock per step).
 struct RefitPanelArgs {
   int rows, n, ld, ng, g, q, rc, np, wdp;
   const float* P;
@@ -205,7 +205,6 @@ struct CdPanelArgs {
   unsigned long long* mid;
   uint32_t* evals;
 };
-bool cd_panel_ok(int n, int sbw);
 hipError_t refit_panel(hipStream_t st, const RefitPanelArgs& a);
 hipError_t cd_panel(hipStream_t st, const CdPanelArgs& a);
 // Folds one pass's logged deltas into the per-chunk loss (exact reference order); nref refit

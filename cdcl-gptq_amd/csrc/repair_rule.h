@@ -34,4 +34,39 @@ inline bool refit_panel_ok(int n, int g, int rows, int cus) {
   return g < n || rows <= 64L * cus;
 }
 
+// Whether the descent may run a KC panel of sub-blocks per launch (k_panel.hip, k_cd_panel) and not a launch
+// pair per sub-block: sub-blocks of 64, or one of all n <= 64. Narrow layers save few launches, and from
+// many rows on lose more in rounds of 16 rows a CU (repair of three passes with the refit: 16384 x 64
+// 0.399 against 0.374 ms a sub-block at a time, 12288 x 64 0.350 and 0.356, 16384 x 128 0.579 and 0.559, 32768 x
+// 256 1.320 and 1.314, 65536 x 256 2.28 and 2.20, 65536 x 512 5.29 and 5.24; 131072 x 1024 27.6 and 28.9).
+inline bool cd_panel_ok(int n, int sbw, int rows, int cus) {
+  if (!(sbw == 64 || (sbw >= n && n <= 64))) return false;
+  return n > 512 || rows <= (n <= 128 ? 48L : 96L) * cus;
+}
+
+// Which of the two a panel takes in one pass: tiles[i] 128-row tiles take part in its i-th of nsub sub-blocks,
+// `both` of them in any, out of np panels. The panel form computes all of its columns' gradient for every
+// such tile, so a sparse selection (refine_frac < 1, chunks that have converged) pays for columns that
+// no row uses; a sub-block at a time computes those alone. In tiles of 128 x 64 times panels (36 ns of the
+// whole device; a launch takes at least half a device of them): the panel form does best while p < q, with
+// what j selected sub-blocks save in sweeps and launches, less what a round of 16-row workgroups adds.
+// Descent alone, two passes, in panels / a sub-block at a time / by this rule: 14336 x 4096, three
+// quarters selected 9.43 / 9.52 / 8.95 ms, a tenth 2.31 / 1.77 / 1.75, 3% 1.51 / 0.85 / 0.86; 4096 x 4096, a quarter
+// 1.36 / 1.40 / 1.20; 1024 x 2048, a tenth 0.237 / 0.296 / 0.224.
+inline bool cd_panel_pays(const int* tiles, int nsub, int both, int np, int rows, int cus) {
+  if (np == 1) return true;  // no gradient of other panels
+  const long least = cus / 2;
+  long j = 0, q = 0;
+  for (int i = 0; i < nsub; ++i) {
+    if (tiles[i] == 0) continue;
+    const long t = (long)tiles[i] * np;
+    q += t > least ? t : least;
+    ++j;
+  }
+  long p = (long)nsub * both * (np - 1);
+  if (p < least) p = least;
+  const long rounds = (rows + 16L * cus - 1) / (16L * cus);
+  return p < q + cus * (2 * j - 3) / 2 - cus * j * rounds / 25;
+}
+
 }  // namespace cdclq

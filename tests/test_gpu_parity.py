@@ -480,6 +480,17 @@ def test_quantize_panel_sweeps(ctx, d_out, n, group):
                     label=f"panel sweeps {d_out}x{n} g{group}, half selected")
 
 
+@pytest.mark.parametrize("d_out,n,frac,rc", [(300, 1300, 0.15, 37), (300, 1300, 0.4, 300), (2100, 800, 0.2, 64),
+                                             (13000, 300, 0.4, 256)])
+def test_quantize_descent_of_a_sparse_selection(ctx, d_out, n, frac, rc):
+    """A pass that takes some KC panels in one launch and others a sub-block at a time: few of the 64-column
+    sub-blocks selected, other ones in each chunk, chunks that converge at different passes, a last panel of
+    one ragged sub-block."""
+    w, x, h, _ = synth_layer(95 + d_out % 7, d_out, n, n + 300)
+    assert_same(*run_both(ctx, w, h, bits=3, group=128, block=128, act_order=False, passes=4, cd_sweeps=2,
+                          refine_frac=frac, row_chunk=rc), label=f"sparse selection {d_out}x{n} {frac}")
+
+
 def test_quantize_descent_fold_of_many_panels(ctx):
     """Gradients of more than 16 KC panels (n = 4608: 18 panels) take the descent form that folds
     the per-panel chains 32 at a time; 2 passes, act-order, against the live oracle."""

@@ -11,6 +11,10 @@ SHIM = """
 using namespace cdclq;
 extern "C" {
 int r_grad_tile(long units, int wd, int cus) { return (int)grad_tile(units, wd, cus); }
+int r_cd_panel_ok(int n, int sbw, int rows, int cus) { return cd_panel_ok(n, sbw, rows, cus); }
+int r_cd_panel_pays(const int* tiles, int nsub, int both, int np, int rows, int cus) {
+  return cd_panel_pays(tiles, nsub, both, np, rows, cus);
+}
 int r_refit_panel_ok(int n, int g, int rows, int cus) { return refit_panel_ok(n, g, rows, cus); }
 }
 """
@@ -52,3 +56,34 @@ def test_refit_by_panels(rules, n, g, most):
     """Groups that fit the panels' pieces take the panel launch while their rows are few rounds of it."""
     for rows in (1, 4096, 8192, 8193, 16384, 16385, 1 << 20):
         assert rules.r_refit_panel_ok(n, g, rows, 256) == (most is None or rows <= most), rows
+
+
+@pytest.mark.parametrize("n,sub_block,most", [(64, 64, 12288), (64, 100, 12288), (40, 40, 12288), (128, 64, 12288),
+                                              (129, 64, 24576), (512, 64, 24576), (513, 64, None), (4096, 64, None),
+                                              (128, 128, 0), (4096, 48, 0), (65, 65, 0)])
+def test_descent_by_panels(rules, n, sub_block, most):
+    for rows in (1, 12288, 12289, 24576, 24577, 1 << 20):
+        assert rules.r_cd_panel_ok(n, sub_block, rows, 256) == (most is None or rows <= most), rows
+
+
+@pytest.mark.parametrize("rows", [1, 256, 1024, 4096, 14336, 32768, 131072])
+@pytest.mark.parametrize("np_", [3, 4, 16, 56])
+def test_descent_panels_of_a_sparse_selection(rules, rows, np_):
+    """A panel whose four sub-blocks every tile selected is one launch; one of them alone, or from 8192 rows on
+    two, take a launch each; of many panels also four that a quarter of the tiles each selected, whose spare
+    columns cost more than three launches."""
+    cus, tiles = 256, -(-rows // 128)
+
+    def pays(t, both):
+        return rules.r_cd_panel_pays((C.c_int * len(t))(*t), len(t), both, np_, rows, cus)
+
+    assert pays([tiles] * 4, tiles)
+    assert not pays([0, 0, tiles, 0], tiles)
+    if rows > 8192:
+        assert not pays([tiles, 0, tiles, 0], tiles)
+        if np_ >= 16:
+            assert not pays([tiles // 4] * 4, tiles)
+
+
+def test_descent_of_one_panel_needs_no_gradient(rules):
+    assert rules.r_cd_panel_pays((C.c_int * 4)(0, 1, 0, 0), 4, 1, 1, 4096, 256)
