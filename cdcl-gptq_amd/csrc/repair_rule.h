@@ -26,11 +26,13 @@ inline GradTile grad_tile(long units, int wd, int cus) {
 // per-group refit keeps two of up to 64, so what it saves in launches it loses again in rounds: groups of
 // two 64-column pieces from the third round on (refit of one pass and the last, groups of 128: 8192 x
 // 2048 3.11 against 3.15 ms, 12288 x 2048 4.46 and 4.10, 14336 x 4096 17.5 and 15.5, 131072 x 512 6.67 and 4.53),
+// in wide layers, where the gradient leaves the launches little, from the second (7000 x 6000 17.9 and 19.3,
+// 5000 x 8192 25.0 and 22.9, 4096 x 8192 18.7 and 19.0),
 // one group alone, which saves a single launch, from the fifth (131072 x 64 0.58 and 0.51; 16384 x 64 0.157 and
 // 0.161); several groups of 64 and less to a panel never (131072 x 256, groups of 16, 7.31 and 7.44).
 inline bool refit_panel_ok(int n, int g, int rows, int cus) {
   if (!(g <= 128 && (g >= n || g == 128 || (g >= 16 && 64 % g == 0)))) return false;
-  if (g > 64) return rows <= 32L * cus;
+  if (g > 64) return rows <= (n <= 6144 ? 32L : 16L) * cus;
   return g < n || rows <= 64L * cus;
 }
 

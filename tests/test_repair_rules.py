@@ -47,14 +47,14 @@ def test_gradient_tile_computes_few_spare_columns(rules, wd):
 
 
 @pytest.mark.parametrize("n,g,most", [  # the most rows on 256 CUs; None: any number
-    (2048, 128, 8192), (128, 128, 8192), (100, 100, 8192), (65, 65, 8192),   # two pieces to a group
+    (2048, 128, 8192), (6144, 128, 8192), (6145, 128, 4096), (128, 128, 8192), (100, 100, 8192), (65, 65, 8192),   # two pieces to a group
     (64, 64, 16384), (20, 20, 16384),                                        # one group, one piece
     (65, 64, None), (2048, 64, None), (2048, 32, None), (300, 16, None),     # groups inside a piece
     (2048, 8, 0), (2048, 96, 0), (2048, 256, 0), (300, 300, 0), (2048, 24, 0),
 ])
 def test_refit_by_panels(rules, n, g, most):
     """Groups that fit the panels' pieces take the panel launch while their rows are few rounds of it."""
-    for rows in (1, 4096, 8192, 8193, 16384, 16385, 1 << 20):
+    for rows in (1, 4096, 4097, 8192, 8193, 16384, 16385, 1 << 20):
         assert rules.r_refit_panel_ok(n, g, rows, 256) == (most is None or rows <= most), rows
 
 
