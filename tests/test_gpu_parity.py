@@ -412,9 +412,9 @@ def test_quantize_repair_knobs(ctx):
 
 @pytest.mark.parametrize("d_out", [1000, 8256, 16450])
 def test_quantize_refit_row_tilings(ctx, d_out):
-    """The group refit takes the smallest workgroups (16, 32 or 64 rows) whose count fits two per
-    CU: on a 256-CU part 1000 rows take the 16-row form, 8256 the 32-row form and 16450 the 64-row
-    form, each with a ragged last workgroup."""
+    """Groups of 128 at the row counts where the refit's form changes on a 256-CU part, each with a ragged last
+    workgroup: 1000 rows run a KC panel of groups per launch, 8256 the per-group refit with 32 rows per
+    workgroup and 16450 with 64, both with whole groups of 16-byte rows."""
     w, x, h, _ = synth_layer(40 + d_out % 7, d_out, 256, 1024)
     assert_same(*run_both(ctx, w, h, bits=4, group=128, block=128, act_order=True, passes=3, row_chunk=64),
                 label=f"refit rows {d_out}")
@@ -442,10 +442,9 @@ def test_quantize_descent_many_rows(ctx):
 
 
 def test_quantize_wide_gradient_tiles(ctx):
-    """128-column repair gradients with at least four (row tile, panel) units per CU take the
-    128 x 128 / 8-wave tile (one E tile read per unit): 131150 rows x 768 columns is 1025 row
-    tiles (ragged last) x 3 panels, and the passes after the first run it over the active
-    tiles' list (or fall back to the 128 x 64 tiles when too few remain)."""
+    """128- and 256-column repair gradients with at least 2.5 tiles of 128 x 128 per CU take those tiles:
+    131150 rows x 768 columns is 1025 row tiles (ragged last) x 3 panels, and the passes after the first
+    run them over the active tiles' list (or the 128 x 64 tiles when too few remain)."""
     w, x, h, _ = synth_layer(47, 131150, 768, 2048)
     assert_same(*run_both(ctx, w, h, bits=4, group=128, block=128, act_order=True, passes=3, row_chunk=64),
                 label="wide gradient tiles")
@@ -471,7 +470,8 @@ def test_quantize_panel_sweeps(ctx, d_out, n, group):
     """The sweeps that run one KC panel of refit groups or descent sub-blocks per launch: 4, 8 and 16
     rows per workgroup (at most 1024, at most 2048 and more rows on a 256-CU part) with a ragged last
     one, groups inside a 64-column piece of H and of two pieces, last panels, pieces and groups of
-    any width, odd n, half of the sub-blocks selected, chunk borders inside a workgroup."""
+    any width, odd n, half of the sub-blocks selected, chunk borders inside a workgroup. (Groups of 8 are
+    too narrow for them: a launch pair per group, beside the descent's panels.)"""
     w, x, h, _ = synth_layer(81 + d_out % 13, d_out, n, n + 200)
     kw = dict(bits=3, group=group, block=128 if group else n, act_order=True, passes=3)
     assert_same(*run_both(ctx, w, h, row_chunk=37, **kw), label=f"panel sweeps {d_out}x{n} g{group}")
@@ -492,11 +492,31 @@ def test_quantize_descent_of_a_sparse_selection(ctx, d_out, n, frac, rc):
 
 
 def test_quantize_descent_fold_of_many_panels(ctx):
-    """Gradients of more than 16 KC panels (n = 4608: 18 panels) take the descent form that folds
-    the per-panel chains 32 at a time; 2 passes, act-order, against the live oracle."""
+    """Gradients of more than 16 KC panels (n = 4608: 18 panels) take the descent forms that keep 32 of
+    the other panels' chains in flight (a panel per launch) and fold 32 at a time (sub-blocks of 48, one
+    per launch, with groups of 96, whose refit folds the 18 panels too); 2 passes, act-order, against the
+    live oracle."""
     w, x, h, _ = synth_layer(71, 96, 4608, 5000)
     assert_same(*run_both(ctx, w, h, bits=4, group=128, block=128, act_order=True, passes=2, row_chunk=32),
                 label="descent fold of 18 panels")
+    assert_same(*run_both(ctx, w, h, bits=4, group=96, block=96, act_order=True, passes=2, row_chunk=32,
+                          sub_block=48), label="descent fold of 18 panels, sub-blocks of 48")
+
+
+@pytest.mark.parametrize("d_out,n,group,block", [
+    (1000, 200, 96, 96), (8256, 200, 96, 96), (16450, 200, 96, 96),  # 16, 32 and 64 rows, a last group of 8
+    (1000, 100, 8, 128), (8256, 100, 8, 128), (16450, 100, 8, 128),
+    (1000, 384, 256, 256),                                           # a whole last group of 128, 16 rows
+    (8256, 255, 128, 128), (16450, 385, 128, 128),                   # groups of 128 off 16 bytes, 32 and 64 rows
+])
+def test_quantize_refit_per_group(ctx, d_out, n, group, block):
+    """The refit of groups of at most 128 columns one launch pair at a time: 16, 32 or 64 rows per
+    workgroup (the smallest whose count fits two per CU, on 256 CUs up to 8192, up to 16384 and more rows)
+    with a ragged last workgroup, on groups that do not tile the KC panels and on more rows than those
+    take; with sub-blocks of 32 the descent folds its chains itself."""
+    w, x, h, _ = synth_layer(23 + d_out % 9, d_out, n, n + 300)
+    assert_same(*run_both(ctx, w, h, bits=3, group=group, block=block, act_order=True, passes=2, row_chunk=64,
+                          sub_block=32), label=f"refit per group {d_out}x{n} g{group}")
 
 
 @pytest.mark.parametrize("block,group,sub_block,mse", [(2048, 128, 1280, False), (1536, 1536, 1100, True),
