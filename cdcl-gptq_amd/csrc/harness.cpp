@@ -201,17 +201,32 @@ int actgen_sample(cdclq_ctx* ctx, ActGen& g, Rng& rng, size_t tokens, float* x) 
   return CDCLQ_OK;
 }
 
-// A dense rows x n operand of the evaluation's tiles: itself, or a copy in `buf` with rows padded to
-// a multiple of 64 floats (*ld the row stride).
-int eval_operand(cdclq_ctx* ctx, DevBuf& buf, const float* src, size_t rows, size_t n, bool direct, const float** out,
-                 long* ld) {
+// `bytes` of scratch for the evaluation: the context's `buf` where they are few or fit what it holds already,
+// else `own`, which goes with the call (operands can be larger than anything the context keeps).
+int eval_scratch(cdclq_ctx* ctx, DevBuf& buf, Dev& own, size_t bytes, float** out) {
+  constexpr size_t kKeep = (size_t)256 << 20;
+  if (bytes <= kKeep || buf.cap >= bytes) {
+    CK(ensure(ctx, buf, bytes));
+    *out = P<float>(buf);
+    return CDCLQ_OK;
+  }
+  HIPCK(own.alloc(bytes));
+  *out = own.as<float>();
+  return CDCLQ_OK;
+}
+
+// A dense rows x n operand of the evaluation's tiles: itself, or a copy in `buf` or `own` with rows padded
+// to a multiple of 64 floats (*ld the row stride).
+int eval_operand(cdclq_ctx* ctx, DevBuf& buf, Dev& own, const float* src, size_t rows, size_t n, bool direct,
+                 const float** out, long* ld) {
   *out = src;
   *ld = (long)n;
   if (direct) return CDCLQ_OK;
   *ld = repair_ld((int)n);
-  CK(ensure(ctx, buf, rows * (size_t)*ld * 4));
-  HIPCK(pad_rows(ctx->st, (long)rows, (int)n, (long)rows, (int)*ld, src, P<float>(buf)));
-  *out = P<float>(buf);
+  float* p;
+  CK(eval_scratch(ctx, buf, own, rows * (size_t)*ld * 4, &p));
+  HIPCK(pad_rows(ctx->st, (long)rows, (int)n, (long)rows, (int)*ld, src, p));
+  *out = p;
   return CDCLQ_OK;
 }
 
@@ -221,13 +236,14 @@ int rel_err_device(cdclq_ctx* ctx, const float* w, const float* wq, const float*
   const bool direct = eval_operand_ok(n, w) && eval_operand_ok(n, wq) && eval_operand_ok(n, x) && eval_operand_ok(n, xt);
   const float *pw, *pq, *px, *pt;
   long ld;
-  CK(eval_operand(ctx, ctx->t1, w, rows, n, direct, &pw, &ld));
-  CK(eval_operand(ctx, ctx->t2, wq, rows, n, direct, &pq, &ld));
-  CK(eval_operand(ctx, ctx->x_in, x, t, n, direct, &px, &ld));
+  Dev ow, oq, ox, ot;
+  CK(eval_operand(ctx, ctx->t1, ow, w, rows, n, direct, &pw, &ld));
+  CK(eval_operand(ctx, ctx->t2, oq, wq, rows, n, direct, &pq, &ld));
+  CK(eval_operand(ctx, ctx->x_in, ox, x, t, n, direct, &px, &ld));
   if (xt == x)
     pt = px;
   else
-    CK(eval_operand(ctx, ctx->y_in, xt, t, n, direct, &pt, &ld));
+    CK(eval_operand(ctx, ctx->y_in, ot, xt, t, n, direct, &pt, &ld));
   CK(ensure(ctx, ctx->proxy_p, eval_partials(rows, t) * 8));
   CK(ensure_pinned(ctx, 16));
   double* sums = static_cast<double*>(ctx->pin);
@@ -326,18 +342,21 @@ int cdclq_proxy_loss_device(cdclq_ctx* ctx, const float* w_t, const float* w_hat
   HIPCK(hipSetDevice(ctx->device));
   const bool direct = eval_operand_ok(n, h);
   const long ld = direct ? (long)n : repair_ld((int)n);
-  CK(ensure(ctx, ctx->t1, rows * (size_t)ld * 4));
-  HIPCK(residual(ctx->st, (int)rows, (int)n, (int)ld, w_t, w_hat, P<float>(ctx->t1)));
+  Dev oe, oh;
+  float* e;
+  CK(eval_scratch(ctx, ctx->t1, oe, rows * (size_t)ld * 4, &e));
+  HIPCK(residual(ctx->st, (int)rows, (int)n, (int)ld, w_t, w_hat, e));
   if (!direct) {  // H with rows (and as many of them as the padded k) of ld floats, zero past n
-    CK(ensure(ctx, ctx->mp, (size_t)ld * ld * 4));
-    HIPCK(pad_rows(ctx->st, (long)n, (int)n, ld, (int)ld, h, P<float>(ctx->mp)));
-    h = P<float>(ctx->mp);
+    float* hp;
+    CK(eval_scratch(ctx, ctx->mp, oh, (size_t)ld * ld * 4, &hp));
+    HIPCK(pad_rows(ctx->st, (long)n, (int)n, ld, (int)ld, h, hp));
+    h = hp;
   }
   CK(ensure(ctx, ctx->proxy_p, eval_partials(rows, n) * 8));
   CK(ensure_pinned(ctx, 16));
   double* sums = static_cast<double*>(ctx->pin);
-  HIPCK(proxy_sum(ctx->st, (int)rows, (int)n, (int)(direct ? n : (n + 31) & ~(size_t)31), P<float>(ctx->t1), ld, h,
-                  ld, P<double>(ctx->proxy_p), sums));
+  HIPCK(proxy_sum(ctx->st, (int)rows, (int)n, (int)(direct ? n : (n + 31) & ~(size_t)31), e, ld, h, ld,
+                  P<double>(ctx->proxy_p), sums));
   HIPCK(hipStreamSynchronize(ctx->st));
   *out = sums[0];
   return CDCLQ_OK;

@@ -115,6 +115,36 @@ def test_proxy_loss_of_an_infinite_residual(ctx, n, off):
         a.free()
 
 
+def _free_bytes():
+    """hipMemGetInfo of the runtime that the library runs on."""
+    so = next(line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64" in line)
+    free, total = cdclq.C.c_size_t(), cdclq.C.c_size_t()
+    assert cdclq.C.CDLL(so).hipMemGetInfo(cdclq.C.byref(free), cdclq.C.byref(total)) == 0
+    return free.value
+
+
+@pytest.mark.parametrize("rows,n,t", [(8, 1001, 150000), (70000, 1001, 9)])
+def test_evaluation_gives_large_copies_back(rows, n, t):
+    """Operands whose rows are padded into copies of over 256 MB: the copies go with the call, only smaller
+    ones stay with the context."""
+    c, L, out = cdclq.Context(0), cdclq.lib(), cdclq.C.c_double()
+    w, x, h = (cdclq.DeviceArray(c, (r, n), np.float32) for r in (rows, t, n))
+    for a in (w, x, h):
+        a.zero()
+    small = cdclq.DeviceArray.from_host(c, np.ones((3, n), np.float32))
+    for _ in range(2):  # the runtime's own allocations come with the first calls
+        c.check(L.cdclq_rel_err_device(c.ptr, small.ptr, small.ptr, small.ptr, small.ptr, 3, n, 3, cdclq.C.byref(out)))
+        c.check(L.cdclq_proxy_loss_device(c.ptr, small.ptr, small.ptr, 3, n, h.ptr, cdclq.C.byref(out)))
+    before = _free_bytes()
+    print(f"[bench] evaluation scratch rows={rows} t={t}", flush=True)
+    c.check(L.cdclq_rel_err_device(c.ptr, w.ptr, w.ptr, x.ptr, x.ptr, rows, n, t, cdclq.C.byref(out)))
+    c.check(L.cdclq_proxy_loss_device(c.ptr, w.ptr, w.ptr, rows, n, h.ptr, cdclq.C.byref(out)))
+    assert before - _free_bytes() <= 64 << 20
+    for a in (w, x, h, small):
+        a.free()
+    c.close()
+
+
 def test_rel_err_refuses_more_tiles_than_a_launch_takes(ctx):
     """2^20 + 1 rows by 131136 tokens are over 2^24 tiles: an error, not the sum of a wrapped launch."""
     rows, n, t = (1 << 20) + 1, 32, 131136
