@@ -389,10 +389,14 @@ int quantize_device(cdclq_ctx* ctx, const float* w, size_t d_out_, size_t n_, co
   unsigned long long* mid = P<unsigned long long>(ctx->mid_d);
   uint32_t* cd_evals = reinterpret_cast<uint32_t*>(mid + MID_SLOTS);
   HIPCK(zero_words(st, reinterpret_cast<int*>(mid), 2 * MID_SLOTS + d_out));
+  const bool do_cd = cfg->refine_frac > 0.0 && cfg->cd_sweeps > 0 && cfg->passes > 0;
+  const bool do_refit = cfg->refit_scales && g <= 1024;
+  const bool repair = cfg->method == CDCLQ_METHOD_CDCL && (do_cd || do_refit);
   // ---- phase 1: blocked GPTQ with lazy updates (src/engine.rs:397-479)
   CK(ensure(ctx, ctx->wwork, wn * 4));
   CK(ensure(ctx, ctx->wq, wn * 4));
-  CK(ensure(ctx, ctx->ebuf, wn * 4));
+  const int lde = repair_ld(n);  // row stride of phase 2's residual, which takes the errors' buffer
+  CK(ensure(ctx, ctx->ebuf, repair ? (size_t)d_out * lde * 4 : wn * 4));
   CK(ensure(ctx, ctx->invd, (size_t)n * 4));
   CK(ensure(ctx, ctx->colloss_d, (size_t)nchunks * n * 8));
   float* wwork = P<float>(ctx->wwork);
@@ -465,9 +469,7 @@ int quantize_device(cdclq_ctx* ctx, const float* w, size_t d_out_, size_t n_, co
   const int n_sb = (n + sbw - 1) / sbw;
   std::vector<double> ld(nchunks, 0.0);
   std::vector<uint64_t> updates(nchunks, 0), refined(nchunks, 0);
-  const bool do_cd = cfg->refine_frac > 0.0 && cfg->cd_sweeps > 0 && cfg->passes > 0;
-  const bool do_refit = cfg->refit_scales && g <= 1024;
-  if (cfg->method == CDCLQ_METHOD_CDCL && (do_cd || do_refit)) {
+  if (repair) {
     PhaseScope ps(ctx, CDCLQ_PHASE_REPAIR);
     std::vector<uint8_t> sel((size_t)nchunks * n_sb, 0);
     if (do_cd) {
@@ -492,9 +494,7 @@ int quantize_device(cdclq_ctx* ctx, const float* w, size_t d_out_, size_t n_, co
     CK(ensure(ctx, ctx->sel_d, sel.size()));
     HIPCK(hipMemcpyAsync(ctx->sel_d.p, sel.data(), sel.size(), hipMemcpyHostToDevice, st));
     // e = W - W_hat (src/engine.rs:516-519), rows of lde floats (phase 1's errors are done with)
-    const int lde = repair_ld(n), kp = (n + 31) & ~31, np = (n + CDCLQ_KC - 1) / CDCLQ_KC;
-    CK(ensure(ctx, ctx->ebuf, (size_t)d_out * lde * 4));
-    eb = P<float>(ctx->ebuf);
+    const int kp = (n + 31) & ~31, np = (n + CDCLQ_KC - 1) / CDCLQ_KC;
     HIPCK(residual(st, d_out, n, lde, wp, wq, eb));
     // steps whose groups / sub-blocks lie inside the KC panels run one panel per launch (repair_rule.h)
     int cus = 0;
