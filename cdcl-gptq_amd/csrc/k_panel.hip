@@ -22,6 +22,7 @@
 // 1.6 ms, 1001 x 1350 11.5 -> 5.1 ms, 2048 x 2048 12.9 -> 8.2 ms, 2048 x 5632 (groups of 64) 68.7 ->
 // 41.8 ms, 4096 x 14336 397 -> 360 ms.
 #include <algorithm>
+#include <cstddef>
 #include <cstdint>
 
 #include "cdclq_dev.h"
@@ -35,6 +36,7 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 constexpr int KC = CDCLQ_KC;
 constexpr int PW = 64;             // columns of a piece of H
 constexpr int PIECE = KC * PW;     // floats of a piece
+constexpr size_t LDS_BYTES = 160 * 1024;
 constexpr int ES = KC + 4;         // row stride of the staged E (16-byte aligned, rows on different banks)
 
 // LDS-only barrier: the wave's LDS writes are visible to the workgroup after it; vector loads and
@@ -191,6 +193,7 @@ __global__ __launch_bounds__(64 * (R < 8 ? 8 : R)) void k_cd_panel(CdPanelArgs a
   __shared__ __align__(16) float Es[R * ES];
   __shared__ float Gs[R * PW];
   __shared__ uint32_t need;
+  static_assert(sizeof(Hs) + sizeof(Es) + sizeof(Gs) + sizeof(need) <= LDS_BYTES, "a CU's LDS");
   const int tid = threadIdx.x, lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = a.n, ld = a.ld, q = a.q, c0 = q * KC;
@@ -366,6 +369,8 @@ __global__ __launch_bounds__(64 * R) void k_refit_panel(RefitPanelArgs a) {
   __shared__ __align__(16) float PH1[PHIN ? 1 : R * PS];
   __shared__ float Zs[R * ZN], snew[R];
   __shared__ int lv[R], mv[R], nlive;
+  static_assert(sizeof(Hs) + sizeof(Es) + sizeof(Cs) + sizeof(PG) + sizeof(PH1) + sizeof(Zs) + sizeof(snew) +
+                        sizeof(lv) + sizeof(mv) + sizeof(nlive) <= LDS_BYTES, "a CU's LDS");
   float* PH = PHIN ? &Hs[1][0] : PH1;          // the products u hu
   const int tid = threadIdx.x, lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -563,7 +568,7 @@ __global__ __launch_bounds__(64 * R) void k_refit_panel(RefitPanelArgs a) {
   }
 }
 
-// rows per workgroup: the smallest whose workgroups (one per CU, 145-163 KB of LDS) fit at once
+// rows per workgroup: the smallest whose workgroups (one per CU) fit at once
 int panel_rows(int rows, int cus) { return rows <= 4 * cus ? 4 : (rows <= 8 * cus ? 8 : 16); }
 
 }  // namespace

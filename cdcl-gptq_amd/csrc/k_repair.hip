@@ -1,11 +1,12 @@
 // Phase-2 kernels (src/engine.rs:534-670): the repair gradient G = E H[:, c0:c0+wd] on the matrix
-// cores, and the refit / coordinate-descent sweeps of groups and sub-blocks that do not lie inside
-// the KC panels (the others run a panel per launch, k_panel.hip).
+// cores, and the refit / coordinate-descent sweeps of one group or sub-block per launch (k_panel.hip runs a
+// KC panel of them per launch; repair_rule.h says which form is taken).
 //
 // Gradient. The reference computes G with matrixmultiply (k = n): per element a fused chain over
 // each KC = 256 panel of k, panels folded in order. The GEMMs compute the panels' chains in
-// parallel with v_mfma_f32_32x32x1_2b_f32 (K = 1, single rounding per product, bit-identical to
-// fmaf) and store the per-panel values; the sweeps (or k_fold) fold them in panel order.
+// parallel, bit-identical to fmaf chains, and store the per-panel values: k_grad on the two-step MFMAs of
+// mfma_tile.h, k_panel_gemm and the lazy updates on v_mfma_f32_32x32x1_2b_f32 (K = 1, a single rounding
+// per product). The sweeps (or k_fold) fold them in panel order.
 //
 // Sweeps. The refit of a group of at most 128 columns computes U H_CC for 16-64 rows on the matrix
 // cores from H_CC staged in LDS (wider groups: one wavefront per row, H_CC from L2). The descent
@@ -330,7 +331,8 @@ typedef MfmaTile<4, 1, 1, 1> GradN;  // 128 x 32, ring of two, 4 workgroups
 // (kfold <= 256: one KC panel), each folded straight into the C values held in registers in k order,
 // C = fma(alpha, chain, C), starting from beta_one ? C : 0 -- one block's update per kfold, several
 // consecutive blocks per launch. Tiles of 128 x 64, wave w rows 32 w .. +31 as one
-// v_mfma_f32_32x32x1_2b accumulator whose blocks are the column halves; E staged as in k_grad, B as
+// v_mfma_f32_32x32x1_2b accumulator whose blocks are the column halves; E staged as [128 rows][8 quads of
+// k], the quad at position p of row r being p ^ (r & 7), B as
 // [32 k][64 cols]; a ring of three with two stages in flight behind the one being multiplied and one
 // bare barrier per stage. A unit covers all of k.
 constexpr int DNB = 3;
@@ -858,7 +860,7 @@ __global__ __launch_bounds__(256) void k_refit_mfma(int rows, int n, int ld, int
       }
     }
   };
-  // whole, 16-byte aligned rows, with chains to fold (the engine always passes them here)
+  // a whole group of 128 columns with chains to fold, in 16-byte aligned rows
   const bool vec = fvec && (n & 3) == 0 && (c0 & 3) == 0;
   if (vec) {  // stage H_CC with 16-byte loads (16 per thread, all in flight) and the codes by words
     // (issued before the fold's first batch, unconditionally in this branch: vector loads complete
