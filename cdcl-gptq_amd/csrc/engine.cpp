@@ -538,7 +538,13 @@ int quantize_device(cdclq_ctx* ctx, const float* w, size_t d_out_, size_t n_, co
       int cnt;
     };
     std::vector<CdStep> steps;
-    std::vector<int> tl((size_t)(1 + n_sb) * ntile), both;
+    // sub-blocks in `grp` consecutive ones each, the KC panels where those may run in one launch: bit i
+    // of cmask[group][chunk] is chunk's selection of the group's i-th
+    const int grp = cpanel ? CDCLQ_KC / 64 : 1, ngrp = (n_sb + grp - 1) / grp;
+    std::vector<uint8_t> cmask((size_t)ngrp * nchunks, 0), tmask(ntile);
+    for (int c = 0; c < nchunks; ++c)
+      for (int s = 0; s < n_sb; ++s) cmask[(size_t)(s / grp) * nchunks + c] |= (uint8_t)(sel[(size_t)c * n_sb + s] << (s % grp));
+    std::vector<int> tl((size_t)(1 + n_sb) * ntile);
     int nl = 0, nt_act = 0;  // lists in use, tiles of list 0
     const size_t apad = ((size_t)nchunks + 15) / 16 * 16, up_bytes = apad + tl.size() * sizeof(int);
     CK(ensure(ctx, ctx->rtiles_d, up_bytes));
@@ -562,46 +568,40 @@ int quantize_device(cdclq_ctx* ctx, const float* w, size_t d_out_, size_t n_, co
       return CDCLQ_OK;
     };
     auto build_tiles = [&]() -> int {
-      // the tiles of chunks that take part (take(chunk)) to tl's next list
-      auto add_list = [&](auto take) -> int {
-        int cnt = 0, *out = tl.data() + (size_t)nl * ntile;
-        for (int t = 0; t < ntile; ++t) {
-          const int c_lo = (t * rt) / rc, c_hi = (std::min((t + 1) * rt, d_out) - 1) / rc;
-          bool need = false;
-          for (int c = c_lo; c <= c_hi && !need; ++c) need = take(c);
-          if (need) out[cnt++] = t;
-        }
-        ++nl;
-        return cnt;
+      // what the active chunks of tile t say of cm[chunk], up to all of `full`
+      // (the device waits for this: at most one look at each chunk per tile and group)
+      auto of_tile = [&](int t, const uint8_t* cm, uint8_t full) {
+        uint8_t m = 0;
+        for (int c = (t * rt) / rc, end = (std::min((t + 1) * rt, d_out) - 1) / rc; c <= end && m != full; ++c)
+          if (act[c]) m |= cm[c];
+        return m;
       };
+      auto next_list = [&]() { return tl.data() + (size_t)nl++ * ntile; };
       nl = 0;
       steps.clear();
-      nt_act = add_list([&](int c) { return act[c] != 0; });
-      const int per = cpanel ? CDCLQ_KC / 64 : 1;
-      for (int s0 = 0; do_cd && s0 < n_sb; s0 += per) {
-        const int l0 = nl, nsub = std::min(per, n_sb - s0);
-        const size_t st0 = steps.size();
-        int cnt[CDCLQ_KC / 64];
-        for (int i = 0; i < nsub; ++i) {
-          cnt[i] = add_list([&](int c) { return act[c] && sel[(size_t)c * n_sb + s0 + i]; });
-          if (cnt[i])
-            steps.push_back({false, s0 + i, nl - 1, cnt[i]});
-          else
-            --nl;
+      int* out = next_list();
+      nt_act = 0;
+      for (int t = 0; t < ntile; ++t)
+        if (of_tile(t, act.data(), 1)) out[nt_act++] = t;
+      for (int q = 0; do_cd && q < ngrp; ++q) {
+        const uint8_t* cm = cmask.data() + (size_t)q * nchunks;
+        const int nsub = std::min(grp, n_sb - q * grp);
+        const uint8_t full = (uint8_t)((1u << nsub) - 1u);
+        int both = 0, cnt[CDCLQ_KC / 64] = {};
+        for (int t = 0; t < ntile; ++t) {
+          const uint8_t m = tmask[t] = of_tile(t, cm, full);
+          both += m != 0;
+          for (int i = 0; i < nsub; ++i) cnt[i] += (m >> i) & 1;
         }
-        if (!cpanel || nl == l0) continue;
-        both.clear();
-        for (size_t k = st0; k < steps.size(); ++k) {
-          const int* l = tl.data() + (size_t)steps[k].list * ntile;
-          const auto mid = both.insert(both.end(), l, l + steps[k].cnt);
-          std::inplace_merge(both.begin(), mid, both.end());
-          both.erase(std::unique(both.begin(), both.end()), both.end());
+        if (!both) continue;
+        const bool panel = cpanel && cd_panel_pays(cnt, nsub, both, np, d_out, cus);
+        for (int i = 0; i < (panel ? 1 : nsub); ++i) {
+          if (!panel && !cnt[i]) continue;
+          steps.push_back({panel, panel ? q : q * grp + i, nl, panel ? both : cnt[i]});
+          out = next_list();
+          for (int t = 0; t < ntile; ++t)
+            if (panel ? tmask[t] != 0 : (tmask[t] >> i) & 1) *out++ = t;
         }
-        if (!cd_panel_pays(cnt, nsub, (int)both.size(), np, d_out, cus)) continue;
-        steps.resize(st0);
-        std::copy(both.begin(), both.end(), tl.begin() + (size_t)l0 * ntile);
-        nl = l0 + 1;
-        steps.push_back({true, s0 / per, l0, (int)both.size()});
       }
       return upload_pass();
     };
