@@ -594,7 +594,7 @@ int quantize_device(cdclq_ctx* ctx, const float* w, size_t d_out_, size_t n_, co
           for (int i = 0; i < nsub; ++i) cnt[i] += (m >> i) & 1;
         }
         if (!both) continue;
-        const bool panel = cpanel && cd_panel_pays(cnt, nsub, both, np, d_out, cus);
+        const bool panel = cpanel && cd_panel_pays(cnt, nsub, both, np, d_out, (int)cfg->cd_sweeps, cus);
         for (int i = 0; i < (panel ? 1 : nsub); ++i) {
           if (!panel && !cnt[i]) continue;
           steps.push_back({panel, panel ? q : q * grp + i, nl, panel ? both : cnt[i]});

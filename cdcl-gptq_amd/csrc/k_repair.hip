@@ -173,8 +173,8 @@ constexpr int DSK = 32;  // k per stage of the direct-to-LDS kernels
 
 // Direct-to-LDS form, used when k % 32 == 0, wd % 4 == 0 and the rows of E and H are 16-byte
 // aligned (k_panel_gemm takes the rest), on the tiles T of mfma_tile.h. The work units are (panel, row
-// tile, column tile), column tiles fastest, panels slowest. XCD x takes the x-th eighth of them and
-// its workgroups (workgroup w runs on XCD w % 8) take them in turn, so that at any time an XCD works on
+// tile, column tile), column tiles fastest, panels slowest. Each XCD takes a run of them, as many as its
+// workgroups (workgroup w runs on XCD w % 8) are of all (grad_share), which take them in turn, so that at any time an XCD works on
 // one or two panels: their rows of H stay in its L2 for every row tile. The persistent grid is
 // sized to the resident workgroup slots and the stage pipeline runs across a workgroup's units.
 //
@@ -197,8 +197,8 @@ __global__ __launch_bounds__(T::THREADS) void k_grad(int m, int wd, int k, const
   const int nct = (wd + T::COLS - 1) / T::COLS;
   const int np = k / CDCLQ_KC + (k % CDCLQ_KC != 0) - (skip >= 0);  // panels computed
   const int nx = min(8, (int)gridDim.x), xcd = blockIdx.x % nx;
-  const int us = ((int)gridDim.x - xcd + nx - 1) / nx;  // workgroups of this XCD
-  const int u0 = (int)((long)xcd * nunits / nx) + (int)blockIdx.x / nx, u1 = (int)((long)(xcd + 1) * nunits / nx);
+  const GradShare sh = grad_share(xcd, (int)gridDim.x, nx, nunits);
+  const int us = sh.stride, u0 = sh.first + (int)blockIdx.x / nx, u1 = sh.end;
   if (u0 >= u1) return;
   const int nrt = nunits / (nct * np);
   const int tid = threadIdx.x, lane = tid & 63;

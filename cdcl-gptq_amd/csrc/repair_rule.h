@@ -11,13 +11,31 @@ enum GradTile { GRAD_128x128, GRAD_128x64, GRAD_64x64, GRAD_128x32 };
 // 5632, 2.6 a CU: 58.1 us against 61.4 on 128 x 64; 5632 x 2048, 2.4 a CU: 57.4 against 52.0) and only where
 // they compute at most a twentieth more columns than the 64-column ones, which is what their rate is ahead; 64
 // x 64 ones where 128 x 64 tiles would leave CUs without one (1001 x 1350: 14.2 against 14.8 us); 128 x 32 ones
-// for 32 columns and fewer (the descent of 8192 x 4096 in sub-blocks of 32, two passes: 10.3 ms against 14.1; of
-// 1024 x 4096, where 64 x 64 tiles are taken: 4.15 ms with either).
+// for 32 columns and fewer while 64 x 64 ones would be more than a CU each (the descent of 8192 x 4096 in
+// sub-blocks of 32, two passes: 10.3 ms against 14.1; the refit of 1920 x 3552 in groups of 8 20.0 against 23.5, of
+// 64 x 3552 18.0 and 17.9).
 inline GradTile grad_tile(long units, int wd, int cus) {
   const long t128 = (wd + 127) / 128, t64 = (wd + 63) / 64;
   if (2 * units * t128 >= 5L * cus && 19 * 2 * t128 <= 20 * t64) return GRAD_128x128;
-  if (units * t64 < cus) return GRAD_64x64;
-  return wd <= 32 ? GRAD_128x32 : GRAD_128x64;
+  if (wd <= 32) return 2 * units > cus ? GRAD_128x32 : GRAD_64x64;
+  return units * t64 >= cus ? GRAD_128x64 : GRAD_64x64;
+}
+
+// The units of an XCD: its workgroups, `stride` of the `grid` (workgroup w runs on XCD w % nx), take units first,
+// first + 1, .. end - 1 in turn. In proportion to the workgroups, not an nx-th each: with a workgroup per unit
+// and a grid that nx does not divide, an XCD would have had more units than workgroups and the launch taken two
+// units' time (64 x 3552 in groups of 8, 28 units: 16.7 us a launch, 9.6 so; the refit of 640 x 1536's descent in
+// sub-blocks of 48 2.38 -> 1.62 ms).
+struct GradShare {
+  int first, end, stride;
+};
+#ifdef __HIP__
+__host__ __device__
+#endif
+inline GradShare grad_share(int xcd, int grid, int nx, int units) {
+  const int per = grid / nx, more = grid % nx;
+  const int w0 = xcd * per + (xcd < more ? xcd : more), n = per + (xcd < more);
+  return {(int)((long)w0 * units / grid), (int)((long)(w0 + n) * units / grid), n};
 }
 
 // Whether the refit of `rows` rows in groups of g runs a KC panel of groups per launch (k_panel.hip,
@@ -50,25 +68,29 @@ inline bool cd_panel_ok(int n, int sbw, int rows, int cus) {
 // `both` of them in any, out of np panels. The panel form computes all of its columns' gradient for every
 // such tile, so a sparse selection (refine_frac < 1, chunks that have converged) pays for columns that
 // no row uses; a sub-block at a time computes those alone. In tiles of 128 x 64 times panels (36 ns of the
-// whole device; a launch takes at least half a device of them): the panel form does best while p < q, with
-// what j selected sub-blocks save in sweeps and launches, less what a round of 16-row workgroups adds.
+// whole device, an eighth more in 64-column launches; a launch takes at least half a device of them): the panel form does best while p < q, with
+// what j selected sub-blocks save in sweeps and launches, less what a round of 16-row workgroups adds, and
+// from the second round on adds again where further sweeps of a sub-block make its rows differ more.
 // Descent alone, two passes, in panels / a sub-block at a time / by this rule: 14336 x 4096, three
 // quarters selected 9.43 / 9.52 / 8.95 ms, a tenth 2.31 / 1.77 / 1.75, 3% 1.51 / 0.85 / 0.86; 4096 x 4096, a quarter
-// 1.36 / 1.40 / 1.20; 1024 x 2048, a tenth 0.237 / 0.296 / 0.224.
-inline bool cd_panel_pays(const int* tiles, int nsub, int both, int np, int rows, int cus) {
+// 1.36 / 1.40 / 1.20; 1024 x 2048, a tenth 0.237 / 0.296 / 0.224. Two sweeps, repair of one pass, in panels / a
+// sub-block at a time: 45528 x 960 5.91 / 5.41, 14336 x 4096 18.9 / 18.5 (ten passes 118.7 / 120.2), 4096 x 1024
+// 1.03 / 1.18.
+inline bool cd_panel_pays(const int* tiles, int nsub, int both, int np, int rows, int sweeps, int cus) {
   if (np == 1) return true;  // no gradient of other panels
   const long least = cus / 2;
   long j = 0, q = 0;
   for (int i = 0; i < nsub; ++i) {
     if (tiles[i] == 0) continue;
     const long t = (long)tiles[i] * np;
-    q += t > least ? t : least;
+    q += t > least ? t + t / 8 : least;
     ++j;
   }
   long p = (long)nsub * both * (np - 1);
   if (p < least) p = least;
   const long rounds = (rows + 16L * cus - 1) / (16L * cus);
-  return p < q + cus * (2 * j - 3) / 2 - cus * j * rounds / 25;
+  const long again = sweeps > 1 ? cus * j * (rounds - 1) / 4 : 0;
+  return p < q + cus * (2 * j - 3) / 2 - cus * j * rounds / 25 - again;
 }
 
 }  // namespace cdclq

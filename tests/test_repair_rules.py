@@ -11,9 +11,21 @@ SHIM = """
 using namespace cdclq;
 extern "C" {
 int r_grad_tile(long units, int wd, int cus) { return (int)grad_tile(units, wd, cus); }
+int r_share_rounds(int grid, int units) {  // every unit once; returns the most that one workgroup takes
+  const int nx = grid < 8 ? grid : 8;
+  int next = 0, most = 0;
+  for (int x = 0; x < nx; ++x) {
+    const GradShare s = grad_share(x, grid, nx, units);
+    if (s.first != next || s.stride != (grid - x + nx - 1) / nx) return -1;
+    next = s.end;
+    const int r = (s.end - s.first + s.stride - 1) / s.stride;
+    most = r > most ? r : most;
+  }
+  return next == units ? most : -1;
+}
 int r_cd_panel_ok(int n, int sbw, int rows, int cus) { return cd_panel_ok(n, sbw, rows, cus); }
-int r_cd_panel_pays(const int* tiles, int nsub, int both, int np, int rows, int cus) {
-  return cd_panel_pays(tiles, nsub, both, np, rows, cus);
+int r_cd_panel_pays(const int* tiles, int nsub, int both, int np, int rows, int sweeps, int cus) {
+  return cd_panel_pays(tiles, nsub, both, np, rows, sweeps, cus);
 }
 int r_refit_panel_ok(int n, int g, int rows, int cus) { return refit_panel_ok(n, g, rows, cus); }
 }
@@ -37,13 +49,24 @@ def test_gradient_tile_computes_few_spare_columns(rules, wd):
     for widths that it divides once it fills the device; 32 columns and fewer take the 32-column tile there."""
     cols = {0: 128, 1: 64, 2: 64, 3: 32}
     least = (wd + 63) // 64 * 64
-    for units in (1, 255, 256, 640, 1792, 100000):
+    for units in (1, 128, 255, 256, 640, 1792, 100000):
         t = rules.r_grad_tile(units, wd, 256)
         assert -(-wd // cols[t]) * cols[t] * 19 <= least * 20, (units, t)
         if wd % 128 == 0 and 2 * units * (wd // 128) >= 5 * 256:
             assert t == 0
         if units >= 256 and wd <= 64:
             assert t == (3 if wd <= 32 else 1)
+        if units <= 128 and wd <= 64:
+            assert t == 2
+
+
+def test_gradient_units_spread_over_the_workgroups(rules):
+    """A workgroup per unit is one round, whatever the count is modulo the XCDs; more units take one round
+    more than their share at most."""
+    for units in [*range(1, 300), 511, 767, 768]:
+        assert rules.r_share_rounds(min(units, 768), units) == 1, units
+    for units in (769, 1000, 1535, 1536, 5000, 24640):
+        assert -(-units // 768) <= rules.r_share_rounds(768, units) <= -(-units // 768) + 1, units
 
 
 @pytest.mark.parametrize("n,g,most", [  # the most rows on 256 CUs; None: any number
@@ -74,10 +97,14 @@ def test_descent_panels_of_a_sparse_selection(rules, rows, np_):
     columns cost more than three launches."""
     cus, tiles = 256, -(-rows // 128)
 
-    def pays(t, both):
-        return rules.r_cd_panel_pays((C.c_int * len(t))(*t), len(t), both, np_, rows, cus)
+    def pays(t, both, sweeps=1):
+        return rules.r_cd_panel_pays((C.c_int * len(t))(*t), len(t), both, np_, rows, sweeps, cus)
 
     assert pays([tiles] * 4, tiles)
+    if rows <= 14336 or np_ > 16:
+        assert pays([tiles] * 4, tiles, 2)  # two sweeps: at few panels not from many rounds of rows on
+    elif rows > 32768 and np_ <= 4:
+        assert not pays([tiles] * 4, tiles, 2)
     assert not pays([0, 0, tiles, 0], tiles)
     if rows > 8192:
         assert not pays([tiles, 0, tiles, 0], tiles)
@@ -86,4 +113,4 @@ def test_descent_panels_of_a_sparse_selection(rules, rows, np_):
 
 
 def test_descent_of_one_panel_needs_no_gradient(rules):
-    assert rules.r_cd_panel_pays((C.c_int * 4)(0, 1, 0, 0), 4, 1, 1, 4096, 256)
+    assert rules.r_cd_panel_pays((C.c_int * 4)(0, 1, 0, 0), 4, 1, 1, 4096, 1, 256)
